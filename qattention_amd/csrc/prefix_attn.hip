@@ -133,18 +133,11 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     constexpr int NI = D / 32;      // 1 KB LDS loads per thread per K (or V) block
     constexpr int RPI = 512 / D;    // key rows per 1 KB load
     static_assert(NI * 4 * 512 == BLK, "a block is 4 waves x NI loads of 1 KB");
-    // Double buffers of the K and V blocks, four LDS variables so that the
-    // compiler tells them apart: a read of one buffer does not wait for the
-    // LDS-DMA loads in flight into another.
-    __shared__ __attribute__((aligned(1024))) uint16_t Kb0[BLK], Kb1[BLK], Vb0[BLK], Vb1[BLK];
+    // Double buffers of the K and V blocks: K 0, K 1, V 0, V 1.
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[4 * BLK];
+    uint16_t *const Kb0 = smem, *const Kb1 = smem + BLK, *const Vb0 = smem + 2 * BLK, *const Vb1 = smem + 3 * BLK;
     // DBG only: the node of each row the epilogue stages in LDS
     __shared__ int32_t dbg_slot[DBG ? 2 * (BLK / D) : 1];
-    auto kbuf = [&](auto i) -> uint16_t* {
-        if constexpr (decltype(i)::value == 0) return Kb0; else return Kb1;
-    };
-    auto vbuf = [&](auto i) -> uint16_t* {
-        if constexpr (decltype(i)::value == 0) return Vb0; else return Vb1;
-    };
 
     // Logical unit order puts the query tiles of one (sequence, kv head, split)
     // next to each other; hardware deals blockIdx round-robin over the 8 XCDs,
@@ -216,37 +209,31 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
 
     // ---- K/V blocks go straight from global memory to LDS (global_load_lds,
     // 16 bytes per lane, lane i of a load writes bytes [16 i, 16 i + 16) of its
-    // 1 KB): load i of wave w covers key rows (w NI + i) RPI .. + RPI - 1, and
-    // each lane fetches the chunk that the swizzle puts at its position ----
-    // Byte offsets of this lane's loads within a block: 32-bit (the host checks
-    // that 64 key rows span less than 4 GB), added to the block's uniform base.
-    uint32_t koff[NI], voff[NI];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const int row = (wave * NI + i) * RPI + lane / DV;
-        const uint32_t col = 16 * ((lane % DV) ^ kv_swz32(row, DV));
-        koff[i] = (uint32_t)row * (uint32_t)kst + col;
-        voff[i] = (uint32_t)row * (uint32_t)vst + col;
-    }
-    auto issue = [&](const char* base, int64_t st, const uint32_t (&off)[NI], int j, uint16_t* buf) {
-        const int kb = k_lo + j * kBN;
+    // 1 KB): load n of wave w covers key rows (w NI + n) RPI .. + RPI - 1, and
+    // each lane fetches the chunk that the swizzle puts at its position.  The
+    // byte offset of a lane's load n within a block is its row's offset plus
+    // colb ^ 16 swz(n RPI) (the swizzle is linear over xor and row n's bits
+    // are disjoint from the lane's), 32-bit (the host checks that 64 key rows
+    // span less than 4 GB), added to the block's uniform base. ----
+    const uint32_t colb = 16 * ((lane % DV) ^ kv_swz32(wave * NI * RPI + lane / DV, DV));
+    const uint32_t krow = (uint32_t)(wave * NI * RPI + lane / DV) * (uint32_t)kst;
+    const uint32_t vrow = (uint32_t)(wave * NI * RPI + lane / DV) * (uint32_t)vst;
+    // First row of block i.  The last block of a range that is no multiple of
+    // 64 keys starts early (its first keys, also in the block before, are
+    // masked), and a block past the end repeats it: every load of the key
+    // loop is of 64 whole rows, without a bound to clamp to.
+    auto block_row = [&](int i) { return min(k_lo + i * kBN, k_hi - kBN); };
+    // a whole block at once, before the loop; block 0 may be the only one and
+    // shorter than 64 rows: rows past the last repeat it
+    auto issue = [&](const char* base, int64_t st, uint32_t row, int i, uint16_t* buf) {
+        const int kb = i == 0 ? k_lo : block_row(i);
+        const uint32_t last = (uint32_t)min(k_hi - 1 - kb, kBN - 1) * (uint32_t)st;
         const char* gb = base + (int64_t)kb * st;
-        if (__builtin_expect(kb + kBN <= k_hi, 1)) {
 #pragma unroll
-            for (int i = 0; i < NI; ++i) lds_dma16(off[i], gb, buf + (wave * NI + i) * 512);
-        } else {
-            // tail block of the split: rows past k_hi - 1 load that key instead
-            const int last = k_hi - 1 - kb;
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int row = (wave * NI + i) * RPI + lane / DV;
-                const uint32_t col = 16 * ((lane % DV) ^ kv_swz32(row, DV));
-                lds_dma16((uint32_t)min(row, last) * (uint32_t)st + col, gb, buf + (wave * NI + i) * 512);
-            }
-        }
+        for (int n = 0; n < NI; ++n)
+            lds_dma16((colb ^ (16 * kv_swz32(n * RPI, DV))) + min(row + (uint32_t)(n * RPI) * (uint32_t)st, last), gb,
+                      buf + (wave * NI + n) * 512);
     };
-    auto issue_k = [&](int j, auto buf) { issue(kbase, kst, koff, j, kbuf(buf)); };
-    auto issue_v = [&](int j, auto buf) { issue(vbase, vst, voff, j, vbuf(buf)); };
 
     // Operand read addresses (elements).  K (A of S^T, step s, key tile t):
     // row 32 t + q32, chunk 2 s + hl: (kaddr0 ^ 16 s) + 32 D t (the swizzle
@@ -263,30 +250,45 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
         vx0 = rx * D + 8 * (cx ^ kv_swz32(rx, DV)) + 4 * (lane & 1);
         vy0 = ry * D + 8 * (cx ^ kv_swz32(ry, DV)) + 4 * (lane & 1);
     }
-
-    // S^T = K Q^T of the block in K buffer buf; step i = (k-step i / 2, key
-    // tile i % 2), so consecutive products write different tiles, and the K
-    // operand of step i + 1 is read before the product of step i is issued.
-    auto s_product = [&](auto buf, f16v_t (&s)[2]) {
-        const uint16_t* kb = kbuf(buf);
+    // LDS byte addresses of this lane's operand reads in K 0 / V 0; buffer,
+    // key tile and 16-key step are immediate offsets.  hide() keeps the
+    // compiler from holding one register per address and buffer, which spills.
+    uint32_t kad[KS], vxa[DT], vya[DT];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+    for (int s = 0; s < KS; ++s) kad[s] = lds0 + 2 * (kaddr0 ^ (16 * s));
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
-        constexpr int NS = 2 * KS;
-        auto fetch = [&](int i) { return ld16(kb + (kaddr0 ^ (16 * (i >> 1))) + 32 * D * (i & 1)); };
-        Vec16 ka[3];
-        ka[0] = fetch(0);
-        ka[1] = fetch(1);
+    for (int dt = 0; dt < DT; ++dt) {
+        vxa[dt] = lds0 + 2 * (vx0 ^ (32 * dt));
+        vya[dt] = lds0 + 2 * (vy0 ^ (32 * dt));
+    }
+    auto hide = [&] {
 #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            if (i + 2 < NS) ka[(i + 2) % 3] = fetch(i + 2);
-            s[i & 1] = mma32<T>(ka[i % 3], qf[i >> 1], s[i & 1]);
-        }
+        for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(kad[s]));
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) asm volatile("" : "+v"(vxa[dt]), "+v"(vya[dt]));
+    };
+    constexpr int NS = 2 * KS;  // products of S^T per block: k-step i / 2, key tile i % 2
+    constexpr int NP = 4 * DT;  // products of O^T per block: 16-key step i / DT, d-tile i % DT
+    constexpr int PF = 3;       // operands read ahead of their product (4 took the split kernel past 256 VGPRs)
+    auto fetch_k = [&](auto buf, int i) {
+        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+        const v4u x = *(__attribute__((address_space(3))) const v4u*)(uintptr_t)(
+            kad[i >> 1] + 2 * (decltype(buf)::value * BLK + 32 * D * (i & 1)));
+        return Vec16{{x[0], x[1], x[2], x[3]}};
+    };
+    auto fetch_v = [&](auto buf, int i) {
+        typedef short v4s __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) v4s* lds_v4s;
+        const uint32_t off = 2 * ((2 + decltype(buf)::value) * BLK + 16 * D * (i / DT));
+        const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(vxa[i % DT] + off));
+        const v4s y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(vya[i % DT] + off));
+        const uint2 x2 = __builtin_bit_cast(uint2, x), y2 = __builtin_bit_cast(uint2, y);
+        return Vec16{{x2.x, x2.y, y2.x, y2.y}};
     };
 
-    // Online softmax of one block (the lane's query; keys 32 t + 8 (r / 4) +
-    // 4 hl + r % 4 of element r of tile t).  The running max is kept on raw
+    // Online softmax (the lane's query; element r of S tile t is key 32 t +
+    // 8 (r / 4) + 4 hl + r % 4 of the block).  The running max is kept on raw
     // scores q.k (scale > 0 keeps the order) and scale*log2(e) is folded into
     // the exponent: p = exp2(s c - m c), one FMA.  Lazy rescaling: the
     // exponent reference m_run only moves when a block max exceeds it by more
@@ -297,138 +299,256 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     // mantissa bits) therefore moves the reference on every new maximum, as
     // the reference's FA2 loop does; fp16 (11 bits) keeps the lazy reference.
     const float csc = p.scale_log2;
-    auto softmax = [&](f16v_t (&s)[2], Vec16 (&pf)[4], float& alpha, bool& rescale, int kb, auto mask_tag) {
-        constexpr bool MASK = decltype(mask_tag)::value;
-        constexpr float kLazy = T::kCode == QATTN_DTYPE_BF16 ? 0.f : 8.f;
-        if constexpr (MASK) {  // tail block of the split: keys at or beyond k_hi do not exist
+    constexpr float kLazy = T::kCode == QATTN_DTYPE_BF16 ? 0.f : 8.f;
+    float mc = 0.f, ps0 = 0.f, ps1 = 0.f;  // m_run csc; the lane's sum of weights, in two parts
+    auto move_ref = [&](float mb) {
+        mb = xor32_max(mb);
+        const bool move = (mb - m_run) * csc > kLazy;  // always true on the first block
+        if (__builtin_expect(__any(move), 0)) {
+            const float m_new = move ? mb : m_run;
+            const float alpha = move ? fast_exp2((m_run - m_new) * csc) : 1.f;  // m_run = -inf: 0
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
+            ps0 *= alpha;
+            ps1 *= alpha;
+            m_run = m_new;
+        }
+        mc = m_run * csc;
+    };
+    // -inf for the keys of a block (first row kb) outside [lo, k_hi)
+    auto mask_block = [&](int kb, int lo, f16v_t (&s)[2]) {
+        if (__builtin_expect(kb < lo || kb + kBN > k_hi, 0)) {
+            int k0 = kb + 4 * hl;
+            asm volatile("" : "+v"(k0));  // (32 key numbers held across the loop would spill)
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (kb + 32 * t + 8 * (r >> 2) + 4 * hl + (r & 3) >= k_hi) s[t][r] = -INFINITY;
+                for (int r = 0; r < 16; ++r) {
+                    const int key = k0 + 32 * t + 8 * (r >> 2) + (r & 3);
+                    if (key < lo || key >= k_hi) s[t][r] = -INFINITY;
+                }
         }
-        float mb = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mb = fmaxf(mb, s[t][r]);
-        mb = xor32_max(mb);
-        const bool move = (mb - m_run) * csc > kLazy;  // always true on the first block
-        const float m_new = move ? mb : m_run;
-        alpha = move ? fast_exp2((m_run - m_new) * csc) : 1.f;  // m_run = -inf: 0
-        rescale |= move;
-        const float mc = m_new * csc;
-        float psum = 0.f;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float e = fast_exp2(__builtin_fmaf(s[t][r], csc, -mc));
-                s[t][r] = e;
-                psum += e;
+    };
+    // One block's 32 weights per lane, element n = 8 th + e of 16-key step th,
+    // in three stages: exponent (0), exponential (1), sum and packing (2).
+    // Stage q of element n runs at step n NT / 32 + q of an iteration's
+    // NS + NP products, so no instruction waits for the one before it and
+    // step th's weights are packed before its first product.
+    constexpr int NT = NS + 3 * DT - 2;
+    Vec16 pf[4];
+    auto stage = [&](f16v_t (&s)[2], int n, int q) {
+        float x = s[n >> 4][n & 15];
+        if (q == 0) x = __builtin_fmaf(x, csc, -mc);
+        if (q == 1) x = fast_exp2(x);
+        s[n >> 4][n & 15] = x;
+        if (q == 2) {
+            if (n & 1) {
+                ps1 += x;
+                pf[n >> 3].w[(n & 7) >> 1] = MfmaOps<T>::pack2(s[n >> 4][(n & 15) - 1], x);
+            } else {
+                ps0 += x;
             }
         }
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
+    };
+    auto weights_at = [&](f16v_t (&s)[2], int i) {
+#pragma unroll
+        for (int q = 2; q >= 0; --q)
+#pragma unroll
+            for (int n = 0; n < 32; ++n)
+                if (n * NT / 32 + q == i) stage(s, n, q);
+    };
+    auto zero = [](f16v_t (&s)[2]) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    pf[2 * t + h].w[i] = MfmaOps<T>::pack2(s[t][8 * h + 2 * i], s[t][8 * h + 2 * i + 1]);
+            for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
     };
-    auto rescale_o = [&](float alpha, bool rescale) {
-        // the accumulators need rescaling only when some running max moved
-        if (__builtin_expect(__any(rescale), 0)) {
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
-        }
+    // Each step of the loop below is kept in its place: the compiler's own
+    // order put the operand reads next to their products and all
+    // exponentials into the PV half.
+    auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+    // All but the N newest DMA loads and every LDS read of this wave are done,
+    // then the workgroup's barrier: what was loaded may be read, what was read
+    // may be overwritten.
+    auto publish = [](auto n) {
+        constexpr int N = decltype(n)::value;
+        __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));  // vmcnt(N) lgkmcnt(0)
+        asm volatile("s_barrier" ::: "memory");
     };
-
-    // O^T += V^T P^T of the block in V buffer buf; step i = (16-key step
-    // i / DT, d-tile i % DT), operands read one step ahead
-    auto pv_product = [&](auto buf, const Vec16 (&pf)[4]) {
-        typedef short v4s __attribute__((ext_vector_type(4)));
-        const uint16_t* vb = vbuf(buf);
-        auto fetch = [&](int i) {
-            const int th = i / DT, dt = i % DT;
-            const uint16_t* ax = vb + (vx0 ^ (32 * dt)) + 16 * D * th;
-            const uint16_t* ay = vb + (vy0 ^ (32 * dt)) + 16 * D * th;
-            const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)ax);
-            const v4s y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)ay);
-            const uint2 x2 = __builtin_bit_cast(uint2, x), y2 = __builtin_bit_cast(uint2, y);
-            return Vec16{{x2.x, x2.y, y2.x, y2.y}};
-        };
-        constexpr int NS = 4 * DT;
-        Vec16 va[3];
-        va[0] = fetch(0);
-        if (NS > 1) va[1] = fetch(1);
-#pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            if (i + 2 < NS) va[(i + 2) % 3] = fetch(i + 2);
-            oacc[i % DT] = mma32<T>(va[i % 3], pf[i / DT], oacc[i % DT]);
-        }
-    };
-
-    // ---- pipeline over the split's blocks j = 0 .. nb-1: iteration j starts
-    // after a barrier that publishes K_{j+1} and V_j, issues V_{j+1} and
-    // K_{j+2} into the buffers freed by the barrier, forms S_{j+1} on the
-    // matrix cores while the softmax of block j runs on the vector ALUs, and
-    // ends with the PV product of block j ----
+    using W0 = std::integral_constant<int, 0>;
+    using W1 = std::integral_constant<int, NI>;
+    using W2 = std::integral_constant<int, 2 * NI>;
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
-    issue_k(0, B0{});
-    issue_v(0, B0{});
-    if (nb > 1) {
-        issue_k(1, B1{});
-        __builtin_amdgcn_s_waitcnt(kWaitVm(NI));  // K_0 and V_0 (and Q) have landed
-    } else {
-        __builtin_amdgcn_s_waitcnt(kWaitVm(0));
-    }
-    __syncthreads();
-    f16v_t sc[2];
-    s_product(B0{}, sc);
-    // block j uses K buffer j & 1 and V buffer j & 1; the loop is unrolled by
-    // two so every buffer choice is a compile-time constant
-    auto step = [&](int j, auto par) {
-        constexpr int P = decltype(par)::value;
-        using Pn = std::integral_constant<int, P ^ 1>;
-        __builtin_amdgcn_s_waitcnt(kWaitVm(0));
-        __syncthreads();
-        issue_v(j + 1, Pn{});
-        if (j + 2 < nb) issue_k(j + 2, par);
-        f16v_t sn[2];
-        Vec16 pf[4];
-        float alpha;
-        bool rescale = false;
-        softmax(sc, pf, alpha, rescale, k_lo + j * kBN, std::false_type{});
-        s_product(Pn{}, sn);
-        rescale_o(alpha, rescale);
-        pv_product(par, pf);
-        sc[0] = sn[0];
-        sc[1] = sn[1];
+    // the DMA loads of an iteration, one at a time: K_{j+3} and V_{j+1}, both
+    // into the buffers of parity B
+    struct Dma {
+        uint32_t col, kr, vr, ld;
+        const char *gk, *gv;
+        int64_t ks, vs;
+        __device__ __forceinline__ void load(uint32_t off, const char*& base, int64_t step, uint32_t lds) {
+            asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
+            base += step;
+        }
+        __device__ __forceinline__ void k(int buf, int n) {
+            load((col ^ (16 * kv_swz32(n * RPI, DV))) + kr, gk, ks, ld + 2 * buf * BLK + n * 1024);
+        }
+        __device__ __forceinline__ void v(int buf, int n) {
+            load((col ^ (16 * kv_swz32(n * RPI, DV))) + vr, gv, vs, ld + 2 * (2 + buf) * BLK + n * 1024);
+        }
     };
-    for (int j = 0; j + 1 < nb; j += 2) {
-        step(j, B0{});
-        if (j + 2 < nb) step(j + 1, B1{});
+    auto dma_of = [&](int j) {
+        Dma d{colb, krow, vrow, lds0 + wave * (NI * 1024), kbase + (int64_t)block_row(j + 3) * kst,
+              vbase + (int64_t)block_row(j + 1) * vst, RPI * kst, RPI * vst};
+        asm volatile("" : "+v"(d.col), "+v"(d.kr), "+v"(d.vr), "+s"(d.ld));  // (as hide())
+        return d;
+    };
+
+    // ---- pipeline over the split's blocks.  Iteration j forms S_{j+1} (NS
+    // products) while the weights of block j are computed, then adds P_j V_j
+    // to O (NP products) while the last of them and the maximum of block j + 1
+    // are.  Its DMA loads are spread between the products (issued together
+    // they hold the wave up for ~500 cycles: the CU takes one 1 KB load per 16
+    // cycles), and each load has a whole iteration to land: the barrier ahead
+    // of the V reads publishes V_j, issued one iteration before, and frees
+    // K_{j+1}'s buffer for K_{j+3}; the one ahead of the next K reads
+    // publishes K_{j+2} and frees V_j's.  Both wait only for the loads older
+    // than the 2 NI newest.
+    //
+    // Two workgroups share a CU; the hardware prefers the older wave, and of
+    // two started together one finished at 50 us and the other, alone, at 69.
+    // Waves in odd iterations run at a higher priority, which keeps the two
+    // side by side (64.5 +- 3 us).
+    //
+    // What bounds it: power.  The chip clocks at 1.62-1.7 GHz in this loop
+    // (2.35 with one workgroup per CU) and a wave pair takes 2770 cycles per
+    // block for 2048 cycles of matrix products; a loop of this instruction
+    // mix without dependencies or waits sustained 80% of the matrix cores at
+    // 1.6 GHz.  The previous form (products and softmax in compiler order, DMA
+    // issued at the top) took 2830-3080 cycles at 1.7-1.75 GHz.
+    // 10240-token prefix, 85 nodes x 4 sequences x 32 / 8 heads, fp16: 84.9 ->
+    // 80.7 us; 4096 shared tokens, 672 x 8 x 32: 416 -> 397; 2048 tokens, 4681 x
+    // 16 x 32: 2.81 -> 2.75 ms. ----
+    issue(kbase, kst, krow, 0, Kb0);
+    issue(vbase, vst, vrow, 0, Vb0);
+    if (nb > 1) {
+        issue(kbase, kst, krow, 1, Kb1);
+        publish(W2{});  // Q and K_0 have landed
+    } else {
+        publish(W1{});
     }
-    {
-        __builtin_amdgcn_s_waitcnt(kWaitVm(0));
-        __syncthreads();
-        const int kb = k_lo + (nb - 1) * kBN;
-        Vec16 pf[4];
-        float alpha;
-        bool rescale = false;
-        if (kb + kBN > k_hi)
-            softmax(sc, pf, alpha, rescale, kb, std::true_type{});
-        else
-            softmax(sc, pf, alpha, rescale, kb, std::false_type{});
-        rescale_o(alpha, rescale);
-        if ((nb - 1) & 1)
-            pv_product(B1{}, pf);
-        else
-            pv_product(B0{}, pf);
+    if (qt * kBM + wave * 32 < rows) {
+        constexpr int AB = NS - (PF < NS ? PF : NS), BB = NP - (PF < NP ? PF : NP);  // steps of the two barriers
+        Vec16 ka[NS - AB], va[NP - BB];
+        constexpr int FK = NS - AB, FV = NP - BB;  // operands ahead
+        auto iter = [&](int j, auto par, f16v_t (&sc)[2], f16v_t (&sn)[2]) {
+            constexpr int P = decltype(par)::value;
+            using Pn = std::integral_constant<int, P ^ 1>;
+            __builtin_amdgcn_s_setprio(P);
+            hide();
+            Dma dma = dma_of(j);
+            fence();
+            zero(sn);
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                if (i == AB) publish(W2{});
+                sn[i & 1] = mma32<T>(ka[i % FK], qf[i >> 1], sn[i & 1]);
+                if (i + FK < NS) ka[i % FK] = fetch_k(Pn{}, i + FK);
+                if (i >= AB && i - AB < FV) va[i - AB] = fetch_v(par, i - AB);
+#pragma unroll
+                for (int n = 0; n < NI; ++n)
+                    if ((AB > 1 ? 1 + n * (AB - 1) / NI : 0) == i) dma.v(P ^ 1, n);
+                weights_at(sc, i);
+                fence();
+            }
+            mask_block(block_row(j + 1), k_lo + (j + 1) * kBN, sn);
+            float mb = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                if (i == BB) publish(W2{});
+                oacc[i % DT] = mma32<T>(va[i % FV], pf[i / DT], oacc[i % DT]);
+                if (i + FV < NP)
+                    va[i % FV] = fetch_v(par, i + FV);
+                else if (i - BB < FK)
+                    ka[i - BB] = fetch_k(par, i - BB);
+#pragma unroll
+                for (int n = 0; n < NI; ++n)
+                    if ((BB > 1 ? 1 + n * (BB - 1) / NI : 0) == i) dma.k(P ^ 1, n);
+                weights_at(sc, NS + i);
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (2 * DT + e * 2 * DT / 16 == i)
+                        mb = fmaxf(fmaxf(mb, sn[e >> 3][2 * (e & 7)]), sn[e >> 3][2 * (e & 7) + 1]);
+                fence();
+            }
+            move_ref(mb);
+            fence();
+        };
+        auto last = [&](auto par, f16v_t (&sc)[2]) {
+            publish(W0{});  // the last V block
+#pragma unroll
+            for (int i = 0; i < FV; ++i) va[i] = fetch_v(par, i);
+#pragma unroll
+            for (int n = 0; n < 32; ++n) {
+                stage(sc, n, 0);
+                stage(sc, n, 1);
+                stage(sc, n, 2);
+            }
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                oacc[i % DT] = mma32<T>(va[i % FV], pf[i / DT], oacc[i % DT]);
+                if (i + FV < NP) va[i % FV] = fetch_v(par, i + FV);
+            }
+        };
+        f16v_t sA[2], sB[2];
+        zero(sA);
+#pragma unroll
+        for (int i = 0; i < FK; ++i) ka[i] = fetch_k(B0{}, i);
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            sA[i & 1] = mma32<T>(ka[i % FK], qf[i >> 1], sA[i & 1]);
+            if (i + FK < NS) ka[i % FK] = fetch_k(B0{}, i + FK);
+        }
+        mask_block(k_lo, k_lo, sA);
+        {
+            float mb = -INFINITY;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mb = fmaxf(fmaxf(mb, sA[e >> 3][2 * (e & 7)]), sA[e >> 3][2 * (e & 7) + 1]);
+            move_ref(mb);
+        }
+        publish(W0{});  // K_0 has been read; V_0 and K_1 have landed
+        if (nb > 2) issue(kbase, kst, krow, 2, Kb0);
+#pragma unroll
+        for (int i = 0; i < FK; ++i) ka[i] = fetch_k(B1{}, i);
+        int j = 0;
+        for (; j + 2 < nb; j += 2) {
+            iter(j, B0{}, sA, sB);
+            iter(j + 1, B1{}, sB, sA);
+        }
+        if (j + 1 < nb) {
+            iter(j, B0{}, sA, sB);
+            last(B1{}, sB);
+        } else {
+            last(B0{}, sA);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        l_run = ps0 + ps1;
+    } else {
+        // a wave past the tile's rows only stages its part of the blocks (672
+        // rows per kv head leave 3 of 24 waves without any: 408 -> 397 us)
+        publish(W0{});
+        if (nb > 2) issue(kbase, kst, krow, 2, Kb0);
+        for (int j = 0; j + 1 < nb; ++j) {
+            Dma dma = dma_of(j);
+            const int buf = (j & 1) ^ 1;
+#pragma unroll
+            for (int n = 0; n < NI; ++n) dma.v(buf, n);
+            publish(W2{});
+#pragma unroll
+            for (int n = 0; n < NI; ++n) dma.k(buf, n);
+            publish(W2{});
+        }
+        publish(W0{});
     }
     __syncthreads();  // the LDS is reused by the fused epilogue
 
