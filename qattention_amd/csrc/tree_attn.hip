@@ -119,6 +119,81 @@ __global__ __launch_bounds__(kThreads) void tree_gather_kernel(TreeParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// Group kernel: the gather walk of GS (2 or 4) q heads of one kv head at once,
+// group_lanes(D) lanes per (token, head group).  The gather kernel loads every
+// ancestor row once per q head, and with grouped heads those loads, not HBM,
+// are its bound (512 bytes per step and query at D = 128 against the row's
+// 512 / (GS x children) from memory); here a loaded row serves GS queries.
+// Few loads in flight per wave and many waves beat the reverse: at D = 128 one
+// step per chunk (K and V: 16 VGPRs) against 2 or 4 steps ran 87.5 / 95 / 105
+// us on 4 x 4681 nodes b=8 32/8 heads, at D = 64 two steps against 4 and 8 ran
+// 64 / 71 / 75 us on 24 ragged trees of up to 1365 nodes 32/8 heads (the
+// gather kernel: 116 and 91 us, the subtree kernel: 126 and 112).
+// ---------------------------------------------------------------------------
+constexpr int group_lanes(int head_dim) { return head_dim == 32 ? 4 : 8; }
+
+// DBG: the walk-export instantiation, as for the gather kernel.
+// hg: Hq / GS, the head groups of a token; pg: GS-head groups per kv head.
+template <typename T, int D, int WALK, int LAYOUT, int GS, bool DBG = false>
+__global__ __launch_bounds__(kThreads) void tree_group_kernel(TreeParams p, Divider hg, Divider pg) {
+    constexpr int LPR = group_lanes(D);
+    constexpr int NCH = D / (8 * LPR);
+    constexpr int SLOTS = kThreads / LPR;
+    constexpr int CH = 2 / NCH;  // walk steps per chunk
+    const int j = threadIdx.x % LPR;
+    const uint32_t nb = gridDim.x, bx = blockIdx.x, per = nb >> 3, rem = nb & 7, x = bx & 7;
+    const uint32_t lbk = x * per + min(x, rem) + (bx >> 3);
+    const int32_t slot = (int32_t)(lbk * SLOTS + threadIdx.x / LPR);  // (the host keeps the grid's slots below 2^31)
+    const int32_t r = divide(slot, hg);
+    const int g = slot - r * hg.d, seq = divide(r, p.msdiv), tok = r - seq * p.max_seqlen;
+    if (seq >= p.B) return;
+    int32_t start, n;
+    if (!seq_bounds(p, seq, start, n)) return;
+    if (tok >= n) return;
+    const int64_t qrow = (int64_t)start + tok;
+    const int h0 = g * GS;
+    Vec16 qf[GS][NCH];
+#pragma unroll
+    for (int u = 0; u < GS; ++u) load_q4<D, false, LPR>(p, seq, qrow, h0 + u, j, qf[u]);
+    float m[GS], l[GS], acc[GS][8 * NCH];
+#pragma unroll
+    for (int u = 0; u < GS; ++u) {
+        m[u] = -INFINITY;
+        l[u] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8 * NCH; ++e) acc[u][e] = 0.f;
+    }
+    const uint16_t* qdummy = (const uint16_t*)p.q + qrow * p.sq_t + (int64_t)h0 * p.sq_h + 8 * j;
+    int32_t* dbg = nullptr;
+    if constexpr (DBG) {
+        if (j == 0) {
+            dbg = p.dbg_walk + (qrow * p.Hq + h0) * (p.max_depth + 1);
+            for (int i = 0; i <= p.max_depth; ++i) dbg[i] = -1;
+        }
+    }
+    Walk4<T, D, WALK, LAYOUT, CH, false, DBG, LPR> w(p, seq, start, n, tok, divide(g, pg), j,
+                                                     LAYOUT == KV_PAGED ? qdummy : nullptr, dbg);
+    do {
+        w.issue();
+#pragma unroll
+        for (int u = 0; u < GS; ++u) w.fold_query(qf[u], m[u], l[u], acc[u]);
+        w.s0 += CH;
+    } while (w.more());
+#pragma unroll
+    for (int u = 0; u < GS; ++u) {
+        if (p.lse)
+            write_out4<T, D, true, false, LPR>(p, seq, qrow, h0 + u, j, m[u], l[u], acc[u]);
+        else
+            write_out4<T, D, false, false, LPR>(p, seq, qrow, h0 + u, j, m[u], l[u], acc[u]);
+    }
+    if constexpr (DBG) {  // the heads of a group share their walk
+        if (j == 0)
+            for (int u = 1; u < GS; ++u)
+                for (int i = 0; i <= p.max_depth; ++i) dbg[u * (p.max_depth + 1) + i] = dbg[i];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Ancestor table kernel (debug export of the walk)
 // ---------------------------------------------------------------------------
 template <int WALK>
@@ -367,6 +442,84 @@ static int gather_dbg(const TreeParams& p, int walk, int layout, bool pstate, hi
                   : launch_gather<T, D, WALK_PARENTS, KV_PACKED, LSE, false, false, true>(p, st);
 }
 
+template <typename T, int D, int WALK, int LAYOUT, int GS>
+static int launch_group_gs(const TreeParams& p, hipStream_t st) {
+    constexpr int SLOTS = kThreads / group_lanes(D);
+    const int64_t blocks = ((int64_t)p.B * p.max_seqlen * (p.Hq / GS) + SLOTS - 1) / SLOTS;
+    const Divider hg = make_divider(p.Hq / GS), pg = make_divider(p.group / GS);
+    if (p.dbg_walk)
+        hipLaunchKernelGGL((tree_group_kernel<T, D, WALK, LAYOUT, GS, true>), dim3((unsigned)blocks), dim3(kThreads), 0,
+                           st, p, hg, pg);
+    else
+        hipLaunchKernelGGL((tree_group_kernel<T, D, WALK, LAYOUT, GS>), dim3((unsigned)blocks), dim3(kThreads), 0, st,
+                           p, hg, pg);
+    return launch_status("tree_group_kernel");
+}
+
+// q heads per slot of the group kernel for a call, or 0: the gather kernel.
+// Its slots must fill the chip: fewer, longer-running waves lose to the gather
+// kernel's one query per slot below about 8 waves per CU for GS = 4 and 16 for
+// GS = 2 (500-node trees b=3, 32/8 heads, D = 128: 1500 waves 13.9 against 12.1
+// us, 2000 15.8 against 17.2, 8000 41.8 against 49.3; D = 64: 2000 waves equal,
+// 3000 12.2 against 13.9; 16/8 heads: 3000 13.5 against 13.0, 4000 16.0 against
+// 17.4).  Packed layouts (cu) without split states only.
+static int group_heads(const TreeParams& p, int head_dim, bool pstate) {
+    const int gs = p.group % 4 == 0 ? 4 : 2;
+    if (!p.cu || pstate || p.group % gs || (int64_t)p.B * p.max_seqlen * p.Hq >= (int64_t(1) << 31)) return 0;
+    const int64_t waves = (int64_t)p.B * p.max_seqlen * (p.Hq / gs) * group_lanes(head_dim) / 64;
+    return waves >= 8192 / gs ? gs : 0;
+}
+
+// Mean walk steps per node of a b-ary heap of n nodes.
+static double heap_steps(int b, int64_t n, int max_depth) {
+    double steps = 0;
+    int64_t first = 0, width = 1;
+    for (int level = 0; first < n; ++level) {
+        steps += (double)std::min(width, n - first) * (std::min(level, max_depth) + 1);
+        if (b == 1 && level >= max_depth) return (steps + (double)(n - first - 1) * (max_depth + 1)) / (double)n;
+        first += width;
+        width = std::min(width * b, n);
+    }
+    return steps / (double)n;
+}
+
+// Whether the subtree kernel is the faster one for a heap walk without split
+// states, from two estimates in us.  A walk costs the bytes its lanes load
+// (each query's Q, O and each slot's K/V row per step) at the rate the
+// vector memory path was seen to reach: 7.2 TB/s for the group kernel, 12.5
+// plus 4 us for the gather kernel.  The subtree kernel costs 5 us plus the
+// larger of its compulsory bytes at 5 TB/s and its rounds of tiles (768
+// workgroups), each 2 us plus 0.07 us per 256 bytes of query rows.  Measured /
+// estimated, subtree against walk: b=4 d=5 x 4, 32 heads 40 / 41 against 48 / 52
+// us; 672 nodes b=28, 32 heads 10.7 / 9.4 against 8.0 / 7.4; 1023 nodes b=2 x 8,
+// 32/8 heads 47 / 54 against 57 / 59; 4681 nodes b=8 x 4, 32/8 heads 126 / 115
+// against 88 / 94; 100 nodes b=4 x 32, 32/8 heads 40 / 33 against 20 / 15.  A
+// gather walk must be clearly cheaper (its rate varies more with the tree).
+static bool subtree_pays(const TreeParams& p, const SubtreePlan& plan, int head_dim, bool paged, int gs) {
+    const double nodes = (double)p.B * p.max_seqlen, row = 2.0 * head_dim;
+    const double steps = heap_steps(p.bdiv.d, p.max_seqlen, p.max_depth);
+    double walk = nodes * (p.Hq / std::max(gs, 1)) * 2 * row * (std::max(gs, 1) + steps) * 1e-6;
+    walk = gs ? walk / 7.2 : 4 + walk / 12.5;
+    if (paged) walk *= 1.15;  // (a page-table round trip per chunk)
+    const double rounds = (double)p.B * p.Hkv * plan.total_tiles / 768;
+    const double qrows = (double)p.max_seqlen * p.group / plan.total_tiles;
+    const double hbm = nodes * 2 * row * (p.Hq + p.Hkv) * 1e-6 / 5.0;
+    const double sub = 5 + std::max(rounds * (2 + 0.07 * qrows * row / 256), hbm);
+    return gs ? sub < walk : 0.85 * sub < walk;
+}
+
+template <typename T, int D>
+static int launch_group(const TreeParams& p, int walk, int layout, hipStream_t st) {
+    if (p.group % 4 == 0) {
+        if (layout == KV_PAGED) return launch_group_gs<T, D, WALK_HEAP, KV_PAGED, 4>(p, st);
+        return walk == WALK_HEAP ? launch_group_gs<T, D, WALK_HEAP, KV_PACKED, 4>(p, st)
+                                 : launch_group_gs<T, D, WALK_PARENTS, KV_PACKED, 4>(p, st);
+    }
+    if (layout == KV_PAGED) return launch_group_gs<T, D, WALK_HEAP, KV_PAGED, 2>(p, st);
+    return walk == WALK_HEAP ? launch_group_gs<T, D, WALK_HEAP, KV_PACKED, 2>(p, st)
+                             : launch_group_gs<T, D, WALK_PARENTS, KV_PACKED, 2>(p, st);
+}
+
 template <typename T, int D>
 static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bool pstate, int algo,
                          hipStream_t st) {
@@ -387,8 +540,11 @@ static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bo
         const int64_t wgs = ok ? (int64_t)p.B * p.Hkv * plan.total_tiles : 0;
         // The subtree kernel needs enough tiles to fill 256 CUs; a merged
         // prefix state makes each query heavier, so it only pays off there
-        // when tiles are plentiful.
-        const bool use = ok && (algo == QATTN_ALGO_SUBTREE || wgs >= (pstate ? 2048 : 512));
+        // when tiles are plentiful.  Without one, the cheaper estimate wins
+        // (uniform batches have no group kernel and keep the tile rule).
+        const bool use = ok && (algo == QATTN_ALGO_SUBTREE ||
+                                (wgs >= (pstate ? 2048 : 512) &&
+                                 (pstate || !p.cu || subtree_pays(p, plan, D, paged, group_heads(p, D, false)))));
         if (algo == QATTN_ALGO_SUBTREE && !ok) {
             if (!paged_ok)
                 set_error("paged subtree kernel: page-table entries %lld (at most %d), page size %d (at most "
@@ -404,6 +560,7 @@ static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bo
         set_error("the subtree kernel supports the heap walk on packed or paged K/V only");
         return QATTN_ERR_ARG;
     }
+    if (group_heads(p, D, pstate)) return launch_group<T, D>(p, walk, layout, st);
     if (p.dbg_walk) {
         // walk export: calls over packed cu_seqlens, either dtype, with or without LSE
         if (!p.cu) {

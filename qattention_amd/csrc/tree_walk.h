@@ -84,13 +84,13 @@ __device__ __forceinline__ void slot_coords(const TreeParams& p, int64_t slot, i
     }
 }
 
-// Q fragment of a query in the 4-lane layout.
-template <int D, bool BATCH = false>
+// Q fragment of a query in the LPR-lane layout (lane j holds chunks j, j + LPR, ...).
+template <int D, bool BATCH = false, int LPR = 4>
 __device__ __forceinline__ void load_q4(const TreeParams& p, int seq, int64_t qrow, int h, int j, Vec16* qf) {
     const uint16_t* qp = (const uint16_t*)p.q + qrow * p.sq_t + (BATCH ? (int64_t)seq * p.sq_b : 0) +
                          (int64_t)h * p.sq_h + 8 * j;
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) qf[i] = ld16(qp + 32 * i);
+    for (int i = 0; i < D / (8 * LPR); ++i) qf[i] = ld16(qp + 8 * LPR * i);
 }
 
 // Initial state from split-K prefix partials (flash-decoding merge of all
@@ -172,13 +172,13 @@ __device__ __forceinline__ void load_partial_state4(const TreeParams& p, int64_t
     }
 }
 
-// Partial dot product of the lane's chunks, reduced over the 4-lane group.
-template <typename T, int NCH>
+// Partial dot product of the lane's chunks, reduced over the LPR-lane group.
+template <typename T, int NCH, int LPR = 4>
 __device__ __forceinline__ float qk4(const Vec16* qf, const Vec16* kf) {
     float d = 0.f;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) d += dot8<T>(qf[i], kf[i]);
-    return group_sum<4>(d);
+    return group_sum<LPR>(d);
 }
 
 // Merge NS scores (log2 domain, -inf = not attended) and their V fragments
@@ -215,9 +215,12 @@ __device__ __forceinline__ void fold_scores(const float* s, const Vec16 (*vf)[NC
 // self-loop).  A caller may issue the first chunk before it builds the
 // initial state, so those loads overlap its own.
 // DBG (walk export): every step's attended node (or -1) is written to dbg[step].
-template <typename T, int D, int WALK, int LAYOUT, int CH_ = 8 / (D / 32), bool BATCH = false, bool DBG = false>
+// LPR: lanes per row (4, or 8 where the loaded rows serve several queries).
+template <typename T, int D, int WALK, int LAYOUT, int CH_ = 8 / (D / 32), bool BATCH = false, bool DBG = false,
+          int LPR = 4>
 struct Walk4 {
-    static constexpr int NCH = D / 32;
+    static constexpr int NCH = D / (8 * LPR);
+    static constexpr int CS = 8 * LPR;  // elements between a lane's chunks
     static constexpr int CH = CH_;  // default 2 steps at D=128: 64 VGPRs of K/V loads in flight per lane
     const TreeParams& p;
     const int seq;
@@ -274,8 +277,8 @@ struct Walk4 {
             const uint16_t* vr = vb + (kvb + row) * p.sv_t;
 #pragma unroll
             for (int i = 0; i < NCH; ++i) {
-                kf[t][i] = ld16(kr + 32 * i);
-                vf[t][i] = ld16(vr + 32 * i);
+                kf[t][i] = ld16(kr + CS * i);
+                vf[t][i] = ld16(vr + CS * i);
             }
             prev = cur;
             if constexpr (WALK == WALK_PARENTS)
@@ -320,22 +323,27 @@ struct Walk4 {
             const uint16_t* vr = ok ? vb + (int64_t)pg[t] * p.sv_page + (int64_t)sl[t] * p.sv_t : qdummy;
 #pragma unroll
             for (int i = 0; i < NCH; ++i) {
-                kf[t][i] = ld16(kr + 32 * i);
-                vf[t][i] = ld16(vr + 32 * i);
+                kf[t][i] = ld16(kr + CS * i);
+                vf[t][i] = ld16(vr + CS * i);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    // Fold the issued chunk into (m, l, acc) and move to the next chunk.
-    __device__ __forceinline__ void fold(const Vec16* qf, float& m, float& l, float* acc) {
+    // Fold the issued chunk into one query's (m, l, acc).
+    __device__ __forceinline__ void fold_query(const Vec16* qf, float& m, float& l, float* acc) {
         float s[CH];
 #pragma unroll
         for (int t = 0; t < CH; ++t) {
-            const float d = qk4<T, NCH>(qf, kf[t]) * p.scale_log2;
+            const float d = qk4<T, NCH, LPR>(qf, kf[t]) * p.scale_log2;
             s[t] = val[t] ? d : -INFINITY;
         }
         fold_scores<T, NCH, CH>(s, vf, m, l, acc);
+    }
+
+    // Fold the issued chunk into (m, l, acc) and move to the next chunk.
+    __device__ __forceinline__ void fold(const Vec16* qf, float& m, float& l, float* acc) {
+        fold_query(qf, m, l, acc);
         s0 += CH;
     }
 
@@ -343,10 +351,10 @@ struct Walk4 {
 };
 
 // Normalise and store one query's output (+ LSE from lane 0 of the group).
-template <typename T, int D, bool LSE, bool BATCH = false>
+template <typename T, int D, bool LSE, bool BATCH = false, int LPR = 4>
 __device__ __forceinline__ void write_out4(const TreeParams& p, int seq, int64_t qrow, int h, int j, float m,
                                            float l, float* acc) {
-    constexpr int NCH = D / 32;
+    constexpr int NCH = D / (8 * LPR);
     // l == 0 only for a query with no attended key; the reference divides by 1
     // there (src/ragged_attn.py:379-380).
     const float l_safe = (l == 0.f) ? 1.f : l;
@@ -358,7 +366,7 @@ __device__ __forceinline__ void write_out4(const TreeParams& p, int seq, int64_t
         float r[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) r[e] = acc[8 * i + e] * inv;
-        st16(optr + 32 * i, pack8<T>(r));
+        st16(optr + 8 * LPR * i, pack8<T>(r));
     }
     if constexpr (LSE) {
         if (j == 0)
