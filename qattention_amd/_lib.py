@@ -148,9 +148,11 @@ def check(rc: int, what: str) -> None:
         raise QAttnError(f"{what} failed: {ERRORS.get(rc, rc)}: {last_error()}")
 
 
+_I64 = {n: C.c_int64 * n for n in (2, 3, 4)}  # (forming the array type costs as much as filling it)
+
+
 def i64arr(vals):
-    arr = (C.c_int64 * len(vals))(*[int(x) for x in vals])
-    return arr
+    return _I64[len(vals)](*map(int, vals))
 
 
 def ptr(t) -> int:

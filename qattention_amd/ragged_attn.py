@@ -52,10 +52,11 @@ def _dtype_code(t: torch.Tensor) -> int:
 def _vec_ok(t: torch.Tensor) -> bool:
     """Rows readable as 16-byte vectors: unit last stride, 8-element aligned
     outer strides, 16-byte aligned base."""
-    if t.numel() == 0:
-        return True
     st = t.stride()
-    return st[-1] == 1 and all(s % 8 == 0 for s in st[:-1]) and t.data_ptr() % 16 == 0
+    outer = 0
+    for s in st[:-1]:
+        outer |= s
+    return (st[-1] == 1 and not outer & 7 and not t.data_ptr() & 15) or t.numel() == 0
 
 
 _LAYOUT_COPIES = [True]
@@ -83,7 +84,7 @@ def _vec(t: torch.Tensor) -> torch.Tensor:
 
 def _require_device(*ts):
     dev = ts[0].device
-    if dev.type != "cuda":
+    if not ts[0].is_cuda:
         raise RuntimeError(
             "qattention_amd runs on a ROCm GPU only (got tensors on "
             f"{dev}); there is no CPU path")
@@ -95,7 +96,26 @@ def _require_device(*ts):
 
 def _stream(device) -> int:
     _lib.ensure_init(device)
-    return torch.cuda.current_stream(device).cuda_stream
+    # (the handle alone: torch.cuda.current_stream builds a Stream object, 1.5 us)
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
+
+
+class _Here:
+    """The current device is the tensors' own: nothing to switch (torch.cuda.device costs 1.2 us)."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def _on(device):
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def _seqlens(cu_seqlens: torch.Tensor, B: int, device, max_seqlen: Optional[int]):
@@ -107,7 +127,7 @@ def _seqlens(cu_seqlens: torch.Tensor, B: int, device, max_seqlen: Optional[int]
     if max_seqlen is None:
         cu_cpu = cu_seqlens.cpu()
         sl = cu_cpu.tolist()
-        max_seqlen = int(max(sl[i + 1] - sl[i] for i in range(B))) if B else 1
+        max_seqlen = int(max([e - b for b, e in zip(sl, sl[1:])])) if B else 1
         cu_dev = cu_cpu.to(device=device, dtype=torch.int32, non_blocking=True)
     else:
         cu_dev = cu_seqlens.to(device=device, dtype=torch.int32, non_blocking=True)
@@ -163,7 +183,7 @@ def _tree_forward(Q, K, V, cu_seqlens, branching_factor: int, max_depth: int,
     LSE = torch.empty(T, Hq, dtype=torch.float32, device=device) if want_lse else None
     scale = 1.0 / math.sqrt(D)
     L = _lib.lib()
-    with torch.cuda.device(device):
+    with _on(device):
         rc = L.qattn_tree_fwd(
             Q.data_ptr(), _lib.i64arr(Q.stride()), K.data_ptr(), _lib.i64arr(K.stride()),
             V.data_ptr(), _lib.i64arr(V.stride()), O.data_ptr(), _lib.i64arr(O.stride()),
@@ -285,7 +305,7 @@ def ragged_attention_with_parents(
         O = torch.empty(Q.shape, dtype=Q.dtype, device=device)
     LSE = torch.empty(T, Hq, dtype=torch.float32, device=device)
     L = _lib.lib()
-    with torch.cuda.device(device):
+    with _on(device):
         rc = L.qattn_tree_parents_fwd(
             Q.data_ptr(), _lib.i64arr(Q.stride()), K.data_ptr(), _lib.i64arr(K.stride()),
             V.data_ptr(), _lib.i64arr(V.stride()), O.data_ptr(), _lib.i64arr(O.stride()),
@@ -341,7 +361,7 @@ def _paged_forward(Q, K_cache, V_cache, page_table, cu_seqlens, branching_factor
         O = torch.empty(Q.shape, dtype=Q.dtype, device=device)
     lse = torch.empty(T, Hq, dtype=torch.float32, device=device) if want_lse else None
     L = _lib.lib()
-    with torch.cuda.device(device):
+    with _on(device):
         rc = L.qattn_tree_paged_fwd(
             Q.data_ptr(), _lib.i64arr(Q.stride()), K_cache.data_ptr(), _lib.i64arr(K_cache.stride()),
             V_cache.data_ptr(), _lib.i64arr(V_cache.stride()), O.data_ptr(), _lib.i64arr(O.stride()),
@@ -409,7 +429,7 @@ def _prefix_tree_forward(Q, K, V, cu_dev, B: int, max_seqlen: int, Kp, kp_stride
             _lib.i64arr(LSE.stride()) if LSE is not None else None, cu_dev.data_ptr())
     sizes = (B, max_seqlen, T, int(tree_seq_stride), int(tree_row0), Hq, Hkv, D)
     tail = (ws.data_ptr(), ws_bytes, int(num_splits), _stream(device))
-    with torch.cuda.device(device):
+    with _on(device):
         if parents is None:
             rc = L.qattn_prefix_tree_fwd(*head, *sizes, int(branching_factor), int(max_depth), 1.0 / math.sqrt(D),
                                          _dtype_code(Q), *tail)
@@ -561,7 +581,7 @@ def prefix_attention(
     lib = _lib.lib()
     ws_bytes = int(lib.qattn_prefix_workspace_bytes(B, ms, T, Hq, Hkv, D, L, int(num_splits))) if T else 0
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         rc = lib.qattn_prefix_fwd(
             Q.data_ptr(), _lib.i64arr(Q.stride()), K_prefix.data_ptr(), _lib.i64arr(kp_stride),
             V_prefix.data_ptr(), _lib.i64arr(vp_stride), L, O.data_ptr(), _lib.i64arr(O.stride()),
@@ -631,7 +651,7 @@ def ragged_tree_attn(
     lib = _lib.lib()
     ws_bytes = int(lib.qattn_prefix_workspace_bytes(B, N, B * N, Hq, Hkv, D, L, int(num_splits))) if B * N else 0
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         rc = lib.qattn_ragged_tree_attn_fwd(
             Q.data_ptr(), _lib.i64arr(Q.stride()), K.data_ptr(), _lib.i64arr(K.stride()),
             V.data_ptr(), _lib.i64arr(V.stride()), O.data_ptr(), _lib.i64arr(O.stride()),
@@ -665,7 +685,7 @@ def fused_lse_merge(
     op, ot = _vec(out_pre), _vec(out_tree)
     result = torch.empty(B, H, Nq, D, dtype=out_pre.dtype, device=device)
     L = _lib.lib()
-    with torch.cuda.device(device):
+    with _on(device):
         rc = L.qattn_lse_merge(
             lse_p.data_ptr(), _lib.i64arr(lse_p.stride()), lse_t.data_ptr(), _lib.i64arr(lse_t.stride()),
             op.data_ptr(), _lib.i64arr(op.stride()), ot.data_ptr(), _lib.i64arr(ot.stride()),
@@ -690,7 +710,7 @@ def ancestor_table(cu_seqlens: torch.Tensor, branching_factor: int, max_depth: i
     if parents is not None:
         par = parents.to(device=device, dtype=torch.int32).contiguous()
     L = _lib.lib()
-    with torch.cuda.device(device):
+    with _on(device):
         rc = L.qattn_ancestors(cu_dev.data_ptr(), _lib.ptr(par), B, ms, T, int(branching_factor),
                                int(max_depth), out.data_ptr(), _stream(device))
     _lib.check(rc, "qattn_ancestors")
