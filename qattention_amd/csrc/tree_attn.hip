@@ -56,16 +56,10 @@ static thread_local int32_t* g_dbg_walk = nullptr;
 // ---------------------------------------------------------------------------
 // DBG: the walk-export instantiation (qattn_debug_walk): every query's walk
 // steps are also written to p.dbg_walk.
-// TPB: threads per workgroup.  A split merge that would occupy under half
-// the CUs (a decode step of a small tree) takes one wave per workgroup
-// instead, so four times the CUs share its loads (each CU's vector memory
-// path, not latency, bounds such a launch: the EAGLE-3 step's merge of 8
-// states over 30 workgroups, 18.62 -> 17.12 us per call).
-template <typename T, int D, int WALK, int LAYOUT, bool LSE, bool PSTATE, bool BATCH, bool DBG = false,
-          int TPB = kThreads>
+template <typename T, int D, int WALK, int LAYOUT, bool LSE, bool PSTATE, bool BATCH, bool DBG = false>
 __global__ __launch_bounds__(kThreads) void tree_gather_kernel(TreeParams p) {
     constexpr int NCH = D / 32;
-    constexpr int SLOTS = TPB / 4;
+    constexpr int SLOTS = kThreads / 4;
     const int j = threadIdx.x & 3;
     // Without split states: XCD-contiguous block order.  The dispatcher
     // places block i on XCD i % 8, so XCD x takes the x-th eighth of the
@@ -190,6 +184,169 @@ __global__ __launch_bounds__(kThreads) void tree_group_kernel(TreeParams p, Divi
         if (j == 0)
             for (int u = 1; u < GS; ++u)
                 for (int i = 0; i <= p.max_depth; ++i) dbg[u * (p.max_depth + 1) + i] = dbg[i];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Split merge and walk of few queries (a decode step of a small tree): one
+// wave per (token, q head), D/8 lanes per row, so the wave's 64 * 8 / D lane
+// groups each take a share of the split states and of the walk's steps and
+// are merged at the end.
+// ---------------------------------------------------------------------------
+// Latency is its bound: the queries are too few to fill the chip, and a query
+// given to 4 lanes runs its 8 states and 8 steps as a chain of round trips.
+// Here the states, the parents (in registers, read by readlane) and then all
+// K/V rows are one round trip each.  One step of a 60-node depth-7 draft tree
+// over 2048 tokens, 32/8 heads, D = 128, 8 splits, both kernels: 4 lanes per
+// query (one-wave workgroups) 16.0 us fp16, 19.0 bf16; 8 lanes 15.2; 16 lanes
+// 13.7; this 13.2 and 14.2.
+constexpr int kMergeParents = 256;
+template <typename T, int D, int WALK, bool BATCH, bool DBG = false>
+__global__ __launch_bounds__(kThreads) void tree_merge_kernel(TreeParams p) {
+    constexpr int LPR = D / 8, NG = 64 / LPR;
+    constexpr bool H = kPartHalf<T>;
+    const int lane = threadIdx.x & 63, j = lane % LPR, g = lane / LPR;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int h, tok, seq;
+    slot_coords(p, (int64_t)blockIdx.x * (kThreads / 64) + wave, (int64_t)gridDim.x * (kThreads / 64), h, tok, seq);
+    if (seq >= p.B) return;
+    int32_t start, n;
+    if (!seq_bounds<BATCH>(p, seq, start, n)) return;
+    if (tok >= n) return;
+    const int64_t qrow = (int64_t)start + tok;
+    const int kvh = h / p.group;
+    // parents 64 i + lane of the sequence
+    const bool regs = WALK == WALK_PARENTS && n <= kMergeParents;
+    const int32_t pb = parents_base<BATCH>(p, seq, start);
+    int32_t pr[kMergeParents / 64] = {};
+    if (regs) {
+#pragma unroll
+        for (int i = 0; i < kMergeParents / 64; ++i)
+            if (64 * i + lane < n) pr[i] = p.parents[pb + 64 * i + lane];
+    }
+    auto next = [&](int32_t cur) {
+        if constexpr (WALK == WALK_HEAP) {
+            return heap_parent(cur, p.bdiv);
+        } else {
+            int32_t par;
+            if (regs) {
+                par = rl(pr[0], cur & 63);
+#pragma unroll
+                for (int i = 1; i < kMergeParents / 64; ++i)
+                    if ((cur >> 6) == i) par = rl(pr[i], cur & 63);
+            } else {
+                par = __builtin_amdgcn_readfirstlane(p.parents[pb + cur]);
+            }
+            return (par >= 0 && par < n) ? par : cur;
+        }
+    };
+    const Vec16 qf = ld16((const uint16_t*)p.q + qrow * p.sq_t + (BATCH ? (int64_t)seq * p.sq_b : 0) +
+                          (int64_t)h * p.sq_h + 8 * j);
+    int32_t* dbg = nullptr;
+    if constexpr (DBG) {
+        if (j == 0) {
+            dbg = p.dbg_walk + (qrow * p.Hq + h) * (p.max_depth + 1);
+            for (int t = g; t <= p.max_depth; t += NG) dbg[t] = -1;
+        }
+    }
+    // ---- this group's split states (numerator / l as stored), two in flight ----
+    float m = -INFINITY, l = 0.f, acc[8] = {};
+    const int64_t plane = p.total_tokens * (int64_t)p.Hq, idx = qrow * p.Hq + h;
+    struct State {
+        float m, l;
+        Vec16 a[H ? 1 : 2];
+    };
+    auto load_state = [&](int s) {
+        State x{};
+        x.m = -INFINITY;
+        if (s < p.n_split) {
+            const int64_t k = s * plane + idx;
+            x.m = p.part_m[k];
+            x.l = p.part_l[k];
+            if constexpr (H) {
+                x.a[0] = ld16((const uint16_t*)p.part_acc + k * D + 8 * j);
+            } else {
+                x.a[0] = ld16((const float*)p.part_acc + k * D + 8 * j);
+                x.a[1] = ld16((const float*)p.part_acc + k * D + 8 * j + 4);
+            }
+        }
+        return x;
+    };
+    auto fold_state = [&](const State& x) {
+        const float mb = fmaxf(m, x.m);
+        if (mb == -INFINITY) return;
+        const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - mb);
+        const float w = x.m == -INFINITY ? 0.f : fast_exp2(x.m - mb) * x.l;
+        l = l * alpha + w;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float v;
+            if constexpr (H)
+                v = elem<F16>(x.a[0], e);
+            else
+                v = __builtin_bit_cast(float, x.a[e >> 2].w[e & 3]);
+            acc[e] = __builtin_fmaf(w, v, acc[e] * alpha);
+        }
+        m = mb;
+    };
+    State st0 = load_state(g), st1 = load_state(NG + g);
+    // ---- the walk: steps t0 + g and t0 + NG + g of each 2 NG are this group's ----
+    const int64_t kvb = kv_base(p, seq, start);
+    const uint16_t* kb = (const uint16_t*)p.k + (int64_t)kvh * p.sk_h + 8 * j;
+    const uint16_t* vb = (const uint16_t*)p.v + (int64_t)kvh * p.sv_h + 8 * j;
+    int32_t cur = tok, prev = -1;
+    for (int t0 = 0; t0 <= p.max_depth && cur != prev; t0 += 2 * NG) {
+        int32_t node[2] = {tok, tok};  // (a step without a key reads the query's own row, score -inf)
+        bool ok[2] = {false, false};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            for (int i = 0; i < NG && t0 + u * NG + i <= p.max_depth && cur != prev; ++i) {
+                if (i == g) {
+                    node[u] = cur;
+                    ok[u] = true;
+                }
+                prev = cur;
+                cur = next(cur);
+            }
+        }
+        Vec16 kf[2], vf[2][1];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            kf[u] = ld16(kb + (kvb + node[u]) * p.sk_t);
+            vf[u][0] = ld16(vb + (kvb + node[u]) * p.sv_t);
+            if constexpr (DBG) {
+                if (j == 0 && ok[u]) dbg[t0 + u * NG + g] = node[u];
+            }
+        }
+        if (t0 == 0) {
+            fold_state(st0);
+            fold_state(st1);
+        }
+        float sc[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const float d = qk4<T, 1, LPR>(&qf, &kf[u]) * p.scale_log2;
+            sc[u] = ok[u] ? d : -INFINITY;
+        }
+        fold_scores<T, 1, 2>(sc, vf, m, l, acc);
+    }
+    for (int s = 2 * NG + g; s < p.n_split; s += NG) fold_state(load_state(s));
+    // ---- merge the groups ----
+#pragma unroll
+    for (int off = LPR; off < 64; off *= 2) {
+        const float mo = __shfl_xor(m, off), lo = __shfl_xor(l, off);
+        const float mb = fmaxf(m, mo);
+        const float a = m == -INFINITY ? 0.f : fast_exp2(m - mb), b = mo == -INFINITY ? 0.f : fast_exp2(mo - mb);
+        l = l * a + lo * b;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = acc[e] * a + __shfl_xor(acc[e], off) * b;
+        m = mb;
+    }
+    if (g == 0) {
+        if (p.lse)
+            write_out4<T, D, true, BATCH, LPR>(p, seq, qrow, h, j, m, l, acc);
+        else
+            write_out4<T, D, false, BATCH, LPR>(p, seq, qrow, h, j, m, l, acc);
     }
 }
 
@@ -408,11 +565,13 @@ static int launch_gather(const TreeParams& p, hipStream_t st) {
         return QATTN_ERR_ARG;
     }
     if constexpr (PSTATE && LAYOUT == KV_PACKED) {
-        if (blocks < 128) {  // (cfg4's merge, 170 workgroups, timed within noise either way)
-            constexpr int S1 = 64 / 4;
-            hipLaunchKernelGGL((tree_gather_kernel<T, D, WALK, LAYOUT, LSE, PSTATE, BATCH, DBG, 64>),
-                               dim3((unsigned)((slots + S1 - 1) / S1)), dim3(64), 0, st, p);
-            return launch_status("tree_gather_kernel");
+        // one wave per query below 8 waves per SIMD (8 x 60 queries x 32 heads:
+        // 41.6 us by the gather kernel, 44.9 by this one; 4 x 60: 43.2 and 40.9)
+        if (slots < 8192) {
+            constexpr int WAVES = kThreads / 64;
+            hipLaunchKernelGGL((tree_merge_kernel<T, D, WALK, BATCH, DBG>),
+                               dim3((unsigned)((slots + WAVES - 1) / WAVES)), dim3(kThreads), 0, st, p);
+            return launch_status("tree_merge_kernel");
         }
     }
     hipLaunchKernelGGL((tree_gather_kernel<T, D, WALK, LAYOUT, LSE, PSTATE, BATCH, DBG>), dim3((unsigned)blocks),
