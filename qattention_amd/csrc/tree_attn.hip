@@ -113,8 +113,8 @@ __global__ __launch_bounds__(kThreads) void tree_gather_kernel(TreeParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Group kernel: the gather walk of GS (2 or 4) q heads of one kv head at once,
-// group_lanes(D) lanes per (token, head group).  The gather kernel loads every
+// Group kernel: the gather walk of GS (1, 2 or 4) q heads of one kv head at
+// once, LPR lanes per (token, head group).  The gather kernel loads every
 // ancestor row once per q head, and with grouped heads those loads, not HBM,
 // are its bound (512 bytes per step and query at D = 128 against the row's
 // 512 / (GS x children) from memory); here a loaded row serves GS queries.
@@ -123,14 +123,16 @@ __global__ __launch_bounds__(kThreads) void tree_gather_kernel(TreeParams p) {
 // us on 4 x 4681 nodes b=8 32/8 heads, at D = 64 two steps against 4 and 8 ran
 // 64 / 71 / 75 us on 24 ragged trees of up to 1365 nodes 32/8 heads (the
 // gather kernel: 116 and 91 us, the subtree kernel: 126 and 112).
+//
+// GS = 1 is the same walk with more lanes per query than the gather kernel's 4,
+// for calls too small to fill the chip with 4.
 // ---------------------------------------------------------------------------
 constexpr int group_lanes(int head_dim) { return head_dim == 32 ? 4 : 8; }
 
 // DBG: the walk-export instantiation, as for the gather kernel.
 // hg: Hq / GS, the head groups of a token; pg: GS-head groups per kv head.
-template <typename T, int D, int WALK, int LAYOUT, int GS, bool DBG = false>
+template <typename T, int D, int WALK, int LAYOUT, int GS, int LPR, bool DBG = false>
 __global__ __launch_bounds__(kThreads) void tree_group_kernel(TreeParams p, Divider hg, Divider pg) {
-    constexpr int LPR = group_lanes(D);
     constexpr int NCH = D / (8 * LPR);
     constexpr int SLOTS = kThreads / LPR;
     constexpr int CH = 2 / NCH;  // walk steps per chunk
@@ -601,32 +603,49 @@ static int gather_dbg(const TreeParams& p, int walk, int layout, bool pstate, hi
                   : launch_gather<T, D, WALK_PARENTS, KV_PACKED, LSE, false, false, true>(p, st);
 }
 
-template <typename T, int D, int WALK, int LAYOUT, int GS>
+template <typename T, int D, int WALK, int LAYOUT, int GS, int LPR>
 static int launch_group_gs(const TreeParams& p, hipStream_t st) {
-    constexpr int SLOTS = kThreads / group_lanes(D);
+    constexpr int SLOTS = kThreads / LPR;
     const int64_t blocks = ((int64_t)p.B * p.max_seqlen * (p.Hq / GS) + SLOTS - 1) / SLOTS;
     const Divider hg = make_divider(p.Hq / GS), pg = make_divider(p.group / GS);
     if (p.dbg_walk)
-        hipLaunchKernelGGL((tree_group_kernel<T, D, WALK, LAYOUT, GS, true>), dim3((unsigned)blocks), dim3(kThreads), 0,
-                           st, p, hg, pg);
+        hipLaunchKernelGGL((tree_group_kernel<T, D, WALK, LAYOUT, GS, LPR, true>), dim3((unsigned)blocks),
+                           dim3(kThreads), 0, st, p, hg, pg);
     else
-        hipLaunchKernelGGL((tree_group_kernel<T, D, WALK, LAYOUT, GS>), dim3((unsigned)blocks), dim3(kThreads), 0, st,
-                           p, hg, pg);
+        hipLaunchKernelGGL((tree_group_kernel<T, D, WALK, LAYOUT, GS, LPR>), dim3((unsigned)blocks), dim3(kThreads), 0,
+                           st, p, hg, pg);
     return launch_status("tree_group_kernel");
 }
 
-// q heads per slot of the group kernel for a call, or 0: the gather kernel.
-// Its slots must fill the chip: fewer, longer-running waves lose to the gather
-// kernel's one query per slot below about 8 waves per CU for GS = 4 and 16 for
-// GS = 2 (500-node trees b=3, 32/8 heads, D = 128: 1500 waves 13.9 against 12.1
-// us, 2000 15.8 against 17.2, 8000 41.8 against 49.3; D = 64: 2000 waves equal,
-// 3000 12.2 against 13.9; 16/8 heads: 3000 13.5 against 13.0, 4000 16.0 against
-// 17.4).  Packed layouts (cu) without split states only.
-static int group_heads(const TreeParams& p, int head_dim, bool pstate) {
-    const int gs = p.group % 4 == 0 ? 4 : 2;
-    if (!p.cu || pstate || p.group % gs || (int64_t)p.B * p.max_seqlen * p.Hq >= (int64_t(1) << 31)) return 0;
-    const int64_t waves = (int64_t)p.B * p.max_seqlen * (p.Hq / gs) * group_lanes(head_dim) / 64;
-    return waves >= 8192 / gs ? gs : 0;
+// q heads per slot and lanes per row of the group kernel for a call; gs 0: the
+// gather kernel.
+struct GroupPlan {
+    int gs, lanes;
+};
+
+// Slots of 2 or 4 heads must fill the chip: fewer, longer-running waves lose to
+// the gather kernel's one query per slot below about 8 waves per CU for GS = 4
+// and 16 for GS = 2 (500-node trees b=3, 32/8 heads, D = 128: 1500 waves 13.9
+// against 12.1 us, 2000 15.8 against 17.2, 8000 41.8 against 49.3; D = 64: 2000
+// waves equal, 3000 12.2 against 13.9; 16/8 heads: 3000 13.5 against 13.0, 4000
+// 16.0 against 17.4).  At the other end the gather kernel's 4 lanes per query
+// leave the chip idle: one 16-byte chunk per lane (D / 8 lanes) ran 60 nodes
+// b=2, 32 heads, D = 128 in 4.75 against 5.76 us, 250 nodes in 5.42 against 6.11,
+// 500 nodes with 32/8 heads in 6.15 against 6.27, and 8 lanes one 672-node b=28
+// tree (3 steps) in 7.5 against 8.8 us, three of them in 16.8 against 17.9, but
+// 1000 nodes b=3 (7 steps) in 12.8 against 12.5.  Packed layouts (cu) without
+// split states only.  steps: walk steps per query, at most.
+static GroupPlan group_plan(const TreeParams& p, int head_dim, int steps, bool pstate) {
+    const int64_t queries = (int64_t)p.B * p.max_seqlen * p.Hq;
+    if (!p.cu || pstate || queries >= (int64_t(1) << 31)) return {0, 0};
+    if (p.group % 2 == 0) {
+        const int gs = p.group % 4 == 0 ? 4 : 2, lanes = group_lanes(head_dim);
+        if (queries / gs * lanes / 64 >= 8192 / gs) return {gs, lanes};
+    }
+    if (head_dim == 32) return {0, 0};
+    if (queries <= (p.group == 1 ? 16384 : 8192)) return {1, head_dim / 8};
+    if (head_dim == 128 && p.group == 1 && queries <= 65536 && steps <= 4) return {1, 8};
+    return {0, 0};
 }
 
 // Mean walk steps per node of a b-ary heap of n nodes.
@@ -658,30 +677,44 @@ static bool subtree_pays(const TreeParams& p, const SubtreePlan& plan, int head_
     const double nodes = (double)p.B * p.max_seqlen, row = 2.0 * head_dim;
     const double steps = heap_steps(p.bdiv.d, p.max_seqlen, p.max_depth);
     double walk = nodes * (p.Hq / std::max(gs, 1)) * 2 * row * (std::max(gs, 1) + steps) * 1e-6;
-    walk = gs ? walk / 7.2 : 4 + walk / 12.5;
+    walk = gs > 1 ? walk / 7.2 : 4 + walk / 12.5;
     if (paged) walk *= 1.15;  // (a page-table round trip per chunk)
     const double rounds = (double)p.B * p.Hkv * plan.total_tiles / 768;
     const double qrows = (double)p.max_seqlen * p.group / plan.total_tiles;
     const double hbm = nodes * 2 * row * (p.Hq + p.Hkv) * 1e-6 / 5.0;
     const double sub = 5 + std::max(rounds * (2 + 0.07 * qrows * row / 256), hbm);
-    return gs ? sub < walk : 0.85 * sub < walk;
+    return gs > 1 ? sub < walk : 0.85 * sub < walk;
+}
+
+template <typename T, int D, int GS, int LPR>
+static int launch_group_walk(const TreeParams& p, int walk, int layout, hipStream_t st) {
+    if (layout == KV_PAGED) return launch_group_gs<T, D, WALK_HEAP, KV_PAGED, GS, LPR>(p, st);
+    return walk == WALK_HEAP ? launch_group_gs<T, D, WALK_HEAP, KV_PACKED, GS, LPR>(p, st)
+                             : launch_group_gs<T, D, WALK_PARENTS, KV_PACKED, GS, LPR>(p, st);
 }
 
 template <typename T, int D>
-static int launch_group(const TreeParams& p, int walk, int layout, hipStream_t st) {
-    if (p.group % 4 == 0) {
-        if (layout == KV_PAGED) return launch_group_gs<T, D, WALK_HEAP, KV_PAGED, 4>(p, st);
-        return walk == WALK_HEAP ? launch_group_gs<T, D, WALK_HEAP, KV_PACKED, 4>(p, st)
-                                 : launch_group_gs<T, D, WALK_PARENTS, KV_PACKED, 4>(p, st);
+static int launch_group(const TreeParams& p, const GroupPlan& gp, int walk, int layout, hipStream_t st) {
+    if (gp.gs == 4) return launch_group_walk<T, D, 4, group_lanes(D)>(p, walk, layout, st);
+    if (gp.gs == 2) return launch_group_walk<T, D, 2, group_lanes(D)>(p, walk, layout, st);
+    if constexpr (D == 128) {
+        if (gp.lanes == 16) return launch_group_walk<T, D, 1, 16>(p, walk, layout, st);
     }
-    if (layout == KV_PAGED) return launch_group_gs<T, D, WALK_HEAP, KV_PAGED, 2>(p, st);
-    return walk == WALK_HEAP ? launch_group_gs<T, D, WALK_HEAP, KV_PACKED, 2>(p, st)
-                             : launch_group_gs<T, D, WALK_PARENTS, KV_PACKED, 2>(p, st);
+    if constexpr (D > 32) return launch_group_walk<T, D, 1, 8>(p, walk, layout, st);
+    set_error("no group kernel for head_dim %d with %d heads per slot", D, gp.gs);  // (not for group_plan's answers)
+    return QATTN_ERR_ARG;
 }
 
 template <typename T, int D>
 static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bool pstate, int algo,
                          hipStream_t st) {
+    // walk steps of a query, at most (a heap of b >= 2: no more than its levels)
+    int steps = p.max_depth < 64 ? p.max_depth + 1 : 64;
+    if (walk == WALK_HEAP && p.bdiv.d > 1) {
+        int levels = 0;
+        for (int64_t first = 0, width = 1; first < p.max_seqlen; first += width, width *= p.bdiv.d) ++levels;
+        steps = std::min(steps, levels);
+    }
     const bool paged = layout == KV_PAGED;
     if (walk == WALK_HEAP && (!paged || !pstate) && algo != QATTN_ALGO_GATHER) {
         SubtreePlan plan;
@@ -703,7 +736,7 @@ static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bo
         // (uniform batches have no group kernel and keep the tile rule).
         const bool use = ok && (algo == QATTN_ALGO_SUBTREE ||
                                 (wgs >= (pstate ? 2048 : 512) &&
-                                 (pstate || !p.cu || subtree_pays(p, plan, D, paged, group_heads(p, D, false)))));
+                                 (pstate || !p.cu || subtree_pays(p, plan, D, paged, group_plan(p, D, steps, false).gs))));
         if (algo == QATTN_ALGO_SUBTREE && !ok) {
             if (!paged_ok)
                 set_error("paged subtree kernel: page-table entries %lld (at most %d), page size %d (at most "
@@ -719,7 +752,8 @@ static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bo
         set_error("the subtree kernel supports the heap walk on packed or paged K/V only");
         return QATTN_ERR_ARG;
     }
-    if (group_heads(p, D, pstate)) return launch_group<T, D>(p, walk, layout, st);
+    const GroupPlan gp = group_plan(p, D, steps, pstate);
+    if (gp.gs) return launch_group<T, D>(p, gp, walk, layout, st);
     if (p.dbg_walk) {
         // walk export: calls over packed cu_seqlens, either dtype, with or without LSE
         if (!p.cu) {

@@ -1,7 +1,8 @@
 """The group kernel: grouped q heads walked together (2 or 4 per loaded K/V row).
 
 It serves packed calls without split states whose slots fill the GPU
-(8192 / GS waves of 64 lanes, GS heads per slot), through the heap walk, the
+(8192 / GS waves of 64 lanes, GS heads per slot), and with one head and more
+lanes per slot those too small to fill it, through the heap walk, the
 explicit-parents walk and paged K/V.  Each case is checked against the fp64
 oracle, O and LSE, and its walk against the oracle's ancestor table; the cases
 just below the threshold run the gather kernel on the same inputs.
@@ -66,6 +67,15 @@ CASES = [
     ([1025, 1024, 7], 2, 3, 16, 8, 128, torch.float16),
     ([2049, 2050], 5, 6, 32, 8, 32, torch.float16),
     ([2100], 1, 9, 32, 8, 64, torch.float16),
+    # one head per slot: 16 and 8 lanes, at and one node past their limits
+    ([512], 2, 9, 32, 32, 128, torch.float16),
+    ([513], 2, 9, 32, 32, 128, torch.bfloat16),
+    ([256, 0], 4, 4, 16, 8, 128, torch.bfloat16),
+    ([257], 4, 4, 32, 8, 64, torch.float16),
+    ([15, 15], 2, 3, 4, 4, 64, torch.float16),
+    ([2048], 28, 3, 32, 32, 128, torch.float16),
+    ([2049], 28, 3, 32, 32, 128, torch.float16),
+    ([1, 3, 0], 3, 2, 3, 1, 128, torch.float16),
 ]
 
 
@@ -150,7 +160,7 @@ def test_group_strided_and_captured():
 
 
 @pytest.mark.parametrize("B,N,b,md,Hq,Hkv,D", [
-    (1, 672, 28, 2, 32, 32, 128),   # auto: the gather walk (one round of wide tiles costs more)
+    (1, 672, 28, 2, 32, 32, 128),   # auto: the walk, 8 lanes per query (one round of wide tiles costs more)
     (4, 1365, 4, 5, 32, 32, 128),   # auto: the subtree kernel
     (24, 341, 4, 4, 32, 8, 64),     # auto: the group kernel
     (8, 1023, 2, 9, 32, 8, 128),    # auto: the subtree kernel, deep trees
