@@ -71,7 +71,7 @@ extern "C" {
 
 /* Kernel selection for qattn_tree_fwd (QATTN_ALGO_AUTO picks per shape). */
 #define QATTN_ALGO_AUTO 0
-#define QATTN_ALGO_GATHER 1  /* one row group per (token, head), gathers from global */
+#define QATTN_ALGO_GATHER 1  /* a row group per (token, head or group of heads), gathers from global */
 #define QATTN_ALGO_SUBTREE 2 /* subtree tiles staged in LDS (heap trees only) */
 
 /* Library version string. */

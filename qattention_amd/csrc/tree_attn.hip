@@ -1,7 +1,7 @@
 // tree_attn.hip -- ancestor-sparse tree-verify attention kernels for gfx950.
 //
-// Two kernels compute the same function (the ancestor walk + softmax of
-// src/ragged_attn.py:262-497):
+// These kernels compute the same function (the ancestor walk + softmax of
+// src/ragged_attn.py:262-497); dispatch_tree picks one:
 //
 //  * tree_gather_kernel   one row group (D/8 lanes, 16 B per lane) per
 //                         (token, q head); the d+1 ancestor rows of a chunk of
@@ -9,6 +9,12 @@
 //                         issued before the first score is formed.  Handles the
 //                         heap walk, the explicit-parent walk and the paged
 //                         K/V layout, and merges split-K prefix partial states.
+//
+//  * tree_group_kernel    the same walk for 2 or 4 q heads of a kv head at
+//                         once, or for one with more lanes per query.
+//
+//  * tree_merge_kernel    merges split-K prefix states and walks, one wave per
+//                         (token, q head), for few queries.
 //
 //  * tree_stream_kernel   heap trees only (subtree_stream.hip).  Persistent
 //                         workgroups walk subtree tiles (a band of BFS levels
