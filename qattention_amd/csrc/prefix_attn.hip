@@ -752,7 +752,7 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
             constexpr int CH1 = 8 / NCH;
             constexpr int CHW = D >= 64 ? CH1 / 2 : CH1;
             using W = Walk4<T, D, WALK, KV_PACKED, CHW, BATCH, DBG>;
-            W w0(tp, seq, s0, n, tokb[0], kvh, j, nullptr, dbg[0]), w1(tp, seq, s0, n, tokb[1], kvh, j, nullptr, dbg[1]);
+            W w0(tp, seq, s0, n, tokb[0], kvh, j, dbg[0]), w1(tp, seq, s0, n, tokb[1], kvh, j, dbg[1]);
             w0.issue();
             w1.issue();
             w0.fold(qf4[0], mw[0], lw[0], acc[0]);

@@ -91,9 +91,6 @@ __global__ __launch_bounds__(kThreads) void tree_gather_kernel(TreeParams p) {
     float m = -INFINITY, l = 0.f, acc[8 * NCH];
     // the first chunk of the walk's K/V loads is in flight while the prefix
     // splits are merged (the walk does not depend on them)
-    // (a paged step without a valid page reads this query's own Q row)
-    const uint16_t* qdummy = (const uint16_t*)p.q + qrow * p.sq_t + (BATCH ? (int64_t)seq * p.sq_b : 0) +
-                             (int64_t)h * p.sq_h + 8 * j;
     int32_t* dbg = nullptr;
     if constexpr (DBG) {
         if (j == 0) {
@@ -101,8 +98,7 @@ __global__ __launch_bounds__(kThreads) void tree_gather_kernel(TreeParams p) {
             for (int i = 0; i <= p.max_depth; ++i) dbg[i] = -1;
         }
     }
-    Walk4<T, D, WALK, LAYOUT, 8 / (D / 32), BATCH, DBG> w(p, seq, start, n, tok, h / p.group, j,
-                                                          LAYOUT == KV_PAGED ? qdummy : nullptr, dbg);
+    Walk4<T, D, WALK, LAYOUT, 8 / (D / 32), BATCH, DBG> w(p, seq, start, n, tok, h / p.group, j, dbg);
     w.issue();
     if constexpr (PSTATE) {
         load_partial_state4<T, D>(p, qrow, h, j, m, l, acc);
@@ -165,7 +161,6 @@ __global__ __launch_bounds__(kThreads) void tree_group_kernel(TreeParams p, Divi
 #pragma unroll
         for (int e = 0; e < 8 * NCH; ++e) acc[u][e] = 0.f;
     }
-    const uint16_t* qdummy = (const uint16_t*)p.q + qrow * p.sq_t + (int64_t)h0 * p.sq_h + 8 * j;
     int32_t* dbg = nullptr;
     if constexpr (DBG) {
         if (j == 0) {
@@ -173,8 +168,7 @@ __global__ __launch_bounds__(kThreads) void tree_group_kernel(TreeParams p, Divi
             for (int i = 0; i <= p.max_depth; ++i) dbg[i] = -1;
         }
     }
-    Walk4<T, D, WALK, LAYOUT, CH, false, DBG, LPR> w(p, seq, start, n, tok, divide(g, pg), j,
-                                                     LAYOUT == KV_PAGED ? qdummy : nullptr, dbg);
+    Walk4<T, D, WALK, LAYOUT, CH, false, DBG, LPR> w(p, seq, start, n, tok, divide(g, pg), j, dbg);
     do {
         w.issue();
 #pragma unroll

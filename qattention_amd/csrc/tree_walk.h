@@ -207,6 +207,13 @@ __device__ __forceinline__ void fold_scores(const float* s, const Vec16 (*vf)[NC
     m = m_new;
 }
 
+// The row that a paged step without a valid page reads: its zeros times the
+// step's weight 0 add nothing for any query that folds the chunk.  (A Q row in
+// its place is only harmless to its own query, not to the other heads of a
+// group: 0 * inf is NaN.)
+// (No const: a constant's address space next to the rows' would make the loads flat ones.)
+static __device__ Vec16 kZeroRow[16];  // 128 elements, the widest head
+
 // The ancestor walk of one query with K/V rows gathered from global memory:
 // steps s = 0..max_depth attend c_s iff c_s != c_{s-1} (src/ragged_attn.py:
 // 338-377 heap, :657-698 parents).  The loads of CH steps are issued together
@@ -229,7 +236,7 @@ struct Walk4 {
     const uint16_t* kb;
     const uint16_t* vb;
     const int32_t tok0;  // the query's own node: the row a step without a key reads
-    const uint16_t* qdummy;  // paged: the query's Q row chunk, read by a step without a valid page
+    const uint16_t* zero;  // this lane's first chunk of kZeroRow
     int32_t cur, prev;
     int s0;
     bool val[CH];
@@ -237,11 +244,11 @@ struct Walk4 {
     int32_t* dbg;  // DBG only: this query's row of the walk export (written by lane 0 of the group)
 
     __device__ __forceinline__ Walk4(const TreeParams& p_, int seq_, int32_t start_, int32_t n_, int tok, int kvh,
-                                     int j, const uint16_t* qdummy_ = nullptr, int32_t* dbg_ = nullptr)
+                                     int j, int32_t* dbg_ = nullptr)
         : p(p_), seq(seq_), pb(parents_base<BATCH>(p_, seq_, start_)), n(n_), kvb(kv_base(p_, seq_, start_)),
           kb((const uint16_t*)p_.k + (int64_t)kvh * p_.sk_h + 8 * j),
-          vb((const uint16_t*)p_.v + (int64_t)kvh * p_.sv_h + 8 * j), tok0(tok), qdummy(qdummy_), cur(tok),
-          prev(-1), s0(0), dbg(dbg_) {}
+          vb((const uint16_t*)p_.v + (int64_t)kvh * p_.sv_h + 8 * j), tok0(tok),
+          zero((const uint16_t*)kZeroRow + 8 * j), cur(tok), prev(-1), s0(0), dbg(dbg_) {}
 
     __device__ __forceinline__ void record(int step, int32_t node) {
         if constexpr (DBG) {
@@ -255,9 +262,8 @@ struct Walk4 {
     // a chunk costs two round trips rather than one per step plus one.
     // K/V loads are unconditional: a step without a key (past max_depth, a
     // stalled walk) reads the query's own row (packed: in bounds and already
-    // attended), or for a paged step without a valid page the query's Q row
-    // (in bounds; finite whenever the output can be), and fold gives it score
-    // -inf (weight 0).  A guarded load would let the compiler move the fold's
+    // attended), or for a paged step without a valid page kZeroRow, and fold
+    // gives it score -inf (weight 0).  A guarded load would let the compiler move the fold's
     // conversions behind each load and wait for it there, one round trip per
     // row.
     __device__ __forceinline__ void issue() {
@@ -294,7 +300,7 @@ struct Walk4 {
     // step's page-table entry is requested before any K/V row and the wait
     // for them leaves no row load behind it (two round trips per chunk).  The
     // entry loads are unconditional too: a logical page past pt_cols reads
-    // the row's last entry (or, for an empty table, the Q row) and is
+    // the row's last entry (or, for an empty table, kZeroRow) and is
     // discarded.
     __device__ __forceinline__ void issue_paged() {
         int32_t pg[CH], sl[CH], nd[CH];
@@ -308,7 +314,7 @@ struct Walk4 {
             okn[t] = okn[t] && lp < p.pt_cols;
             const int32_t* ent = p.pt_cols > 0
                                      ? p.page_table + (int64_t)seq * p.pt_cols + min(lp, p.pt_cols - 1)
-                                     : (const int32_t*)qdummy;
+                                     : (const int32_t*)zero;
             pg[t] = *ent;
             prev = cur;
             cur = walk_next<WALK>(p, pb, n, cur);
@@ -319,8 +325,8 @@ struct Walk4 {
             const bool ok = okn[t] && pg[t] >= 0 && pg[t] < p.num_pages;
             val[t] = ok;
             record(s0 + t, ok ? nd[t] : -1);
-            const uint16_t* kr = ok ? kb + (int64_t)pg[t] * p.sk_page + (int64_t)sl[t] * p.sk_t : qdummy;
-            const uint16_t* vr = ok ? vb + (int64_t)pg[t] * p.sv_page + (int64_t)sl[t] * p.sv_t : qdummy;
+            const uint16_t* kr = ok ? kb + (int64_t)pg[t] * p.sk_page + (int64_t)sl[t] * p.sk_t : zero;
+            const uint16_t* vr = ok ? vb + (int64_t)pg[t] * p.sv_page + (int64_t)sl[t] * p.sv_t : zero;
 #pragma unroll
             for (int i = 0; i < NCH; ++i) {
                 kf[t][i] = ld16(kr + CS * i);
