@@ -186,10 +186,12 @@ __device__ __forceinline__ float qk4(const Vec16* qf, const Vec16* kf) {
 template <typename T, int NCH, int NS>
 __device__ __forceinline__ void fold_scores(const float* s, const Vec16 (*vf)[NCH], float& m, float& l,
                                             float* acc) {
+    // (a maximum that a NaN passes through: fmaxf would drop a chunk of nothing
+    // but NaN scores as one without keys)
     float cm = s[0];
 #pragma unroll
-    for (int t = 1; t < NS; ++t) cm = fmaxf(cm, s[t]);
-    const float m_new = fmaxf(m, cm);
+    for (int t = 1; t < NS; ++t) cm = __builtin_elementwise_maximum(cm, s[t]);
+    const float m_new = __builtin_elementwise_maximum(m, cm);
     if (m_new == -INFINITY) return;  // nothing attended yet
     if (m != -INFINITY) {
         const float alpha = fast_exp2(m - m_new);

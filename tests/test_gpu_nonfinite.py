@@ -48,3 +48,57 @@ def test_paged_heads_of_a_group_are_independent(D, Hkv, b, md):
             O2, L2 = call(q2)
             keep = [i for i in range(Hq) if i % g != h]
             assert torch.equal(O2[:, keep], O[:, keep]) and torch.equal(L2[:, keep], L[:, keep]), (bad, h)
+
+
+def _attends(cu, b, md, parents, node):
+    """Tokens of the first sequence's batch row whose walk attends its node `node`."""
+    from oracle import clib
+    anc = (clib.ancestor_table_heap(cu.numpy(), b, md) if parents is None
+           else clib.ancestor_table_parents(cu.numpy(), parents, md))
+    first = np.zeros(anc.shape[0], dtype=bool)
+    first[: int(cu[1])] = True
+    return torch.from_numpy((anc == node).any(1) & first)
+
+
+@pytest.mark.parametrize("walk", ["heap", "parents", "paged"])
+@pytest.mark.parametrize("lens,Hq,Hkv,D", [
+    ([2048, 30], 32, 8, 128),   # 4 heads per slot, one step per chunk
+    ([2100, 30], 32, 16, 128),  # 2 heads per slot
+    ([2100, 30], 32, 8, 64),    # 4 heads, two steps per chunk
+    ([500], 32, 32, 128),       # one head, 16 lanes
+    ([200], 32, 32, 64),        # one head, 8 lanes
+    ([1500], 32, 32, 128),      # gather kernel
+])
+def test_nan_key_reaches_who_attends_it(lens, Hq, Hkv, D, walk):
+    """NaN in a leaf's, an inner node's and a root's K row (of different kv heads):
+    exactly the queries that attend the node become NaN, O and LSE."""
+    from qattention_amd import _lib, ragged_attn as ra
+    b, md = 4, 6
+    Q, K, V, cu = make_inputs(lens, Hq, D, 9100 + D + Hkv, Hkv=Hkv)
+    par = None
+    if walk == "parents":
+        par = np.concatenate([np.maximum(np.arange(n) - 1, 0) // b for n in lens]).astype(np.int32)
+    nodes = [lens[0] - 1, 6, 0]
+    K2 = K.clone()
+    for h, node in enumerate(nodes):
+        K2[node, h, 1] = float("nan")
+
+    def call(k):
+        q, k, v = Q.to(DEV), k.to(DEV), V.to(DEV)
+        if walk == "heap":
+            return ra._tree_forward(q, k, v, cu, b, md, max(lens), True, _lib.ALGO_GATHER)
+        if walk == "parents":
+            return ra.ragged_attention_with_parents(q, k, v, cu, torch.from_numpy(par).to(DEV), md, max(lens))
+        Kc, Vc, pt = ra.build_paged_kv(list(k.split(lens)), list(v.split(lens)), 16)
+        return ra._paged_forward(q, Kc, Vc, pt.to(DEV), cu, b, md, max(lens), True, _lib.ALGO_GATHER)
+
+    say("nan key", walk, lens, Hq, Hkv, D)
+    (O, L), (O2, L2) = call(K), call(K2)
+    g = Hq // Hkv
+    hit = torch.zeros(Q.shape[0], Hq, dtype=torch.bool)
+    for h, node in enumerate(nodes):
+        hit[:, h * g:(h + 1) * g] = _attends(cu, b, md, par, node)[:, None]
+    hit = hit.to(DEV)
+    assert torch.equal(torch.isnan(L2), hit)
+    assert torch.equal(torch.isnan(O2).all(-1), hit) and torch.equal(torch.isnan(O2).any(-1), hit)
+    assert torch.equal(O2[~hit], O[~hit]) and torch.equal(L2[~hit], L[~hit])
