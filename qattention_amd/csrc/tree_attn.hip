@@ -275,10 +275,11 @@ __global__ __launch_bounds__(kThreads) void tree_merge_kernel(TreeParams p) {
         return x;
     };
     auto fold_state = [&](const State& x) {
+        // (a split of nothing but NaN scores has m = -inf and l = NaN: its
+        // weight 0 * l carries the NaN on)
         const float mb = fmaxf(m, x.m);
-        if (mb == -INFINITY) return;
         const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - mb);
-        const float w = x.m == -INFINITY ? 0.f : fast_exp2(x.m - mb) * x.l;
+        const float w = (x.m == -INFINITY ? 0.f : fast_exp2(x.m - mb)) * x.l;
         l = l * alpha + w;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {

@@ -102,3 +102,36 @@ def test_nan_key_reaches_who_attends_it(lens, Hq, Hkv, D, walk):
     assert torch.equal(torch.isnan(L2), hit)
     assert torch.equal(torch.isnan(O2).all(-1), hit) and torch.equal(torch.isnan(O2).any(-1), hit)
     assert torch.equal(O2[~hit], O[~hit]) and torch.equal(L2[~hit], L[~hit])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,Hq,Hkv,D", [
+    (60, 16, 4, 128),   # one wave per query
+    (60, 16, 4, 64),
+    (600, 16, 4, 128),  # gather kernel
+])
+def test_nan_split_reaches_its_heads(N, Hq, Hkv, D, dtype):
+    """NaN in every key of one of ten splits, in one key of another, or in a tree
+    row: the kv head's queries (that attend it) become NaN, the others stay."""
+    from qattention_amd import ragged_attn as ra
+    b, md, L, ns = 3, 5, 640, 10
+    Q, K, V, cu = make_inputs([N], Hq, D, 9200 + D + N, dtype=dtype, Hkv=Hkv)
+    g = torch.Generator().manual_seed(9201)
+    Kp, Vp = (torch.randn(1, L, Hkv, D, generator=g).to(dtype) for _ in range(2))
+    call = lambda k, kp: ra.ragged_attention_prefix(  # noqa: E731
+        *(x.to(DEV) for x in (Q, k, V, cu, kp, Vp)), b, md, max_seqlen=N, return_lse=True, num_splits=ns)
+    say("nan split", N, Hq, Hkv, D, dtype)
+    O, lse = call(K, Kp)
+    K2, Kp2 = K.clone(), Kp.clone()
+    Kp2[0, 64:128, 0, 1] = float("nan")
+    Kp2[0, 600, 1, 1] = float("nan")
+    K2[7, 2, 1] = float("nan")
+    O2, lse2 = call(K2, Kp2)
+    r = Hq // Hkv
+    hit = torch.zeros(N, Hq, dtype=torch.bool)
+    hit[:, :2 * r] = True
+    hit[:, 2 * r:3 * r] = _attends(cu, b, md, None, 7)[:, None]
+    hit = hit.to(DEV)
+    assert torch.equal(torch.isnan(lse2), hit)
+    assert torch.equal(torch.isnan(O2).all(-1), hit) and torch.equal(torch.isnan(O2).any(-1), hit)
+    assert torch.equal(O2[~hit], O[~hit]) and torch.equal(lse2[~hit], lse[~hit])
