@@ -171,6 +171,8 @@ __global__ __launch_bounds__(kThreads) void tree_group_kernel(TreeParams p, Divi
     Walk4<T, D, WALK, LAYOUT, CH, false, DBG, LPR> w(p, seq, start, n, tok, divide(g, pg), j, dbg);
     do {
         w.issue();
+        // (more tokens share a wave than in the gather kernel, so shorter walks wait for longer ones)
+        if constexpr (GS > 1 && LAYOUT == KV_PACKED) w.drop_invalid();
 #pragma unroll
         for (int u = 0; u < GS; ++u) w.fold_query(qf[u], m[u], l[u], acc[u]);
         w.s0 += CH;
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(kThreads) void tree_merge_kernel(TreeParams p) {
             const float d = qk4<T, 1, LPR>(&qf, &kf[u]) * p.scale_log2;
             sc[u] = ok[u] ? d : -INFINITY;
         }
-        fold_scores<T, 1, 2>(sc, vf, m, l, acc);
+        if (ok[0]) fold_scores<T, 1, 2, true>(sc, vf, m, l, acc, ok);
     }
     for (int s = 2 * NG + g; s < p.n_split; s += NG) fold_state(load_state(s));
     // ---- merge the groups ----

@@ -183,9 +183,11 @@ __device__ __forceinline__ float qk4(const Vec16* qf, const Vec16* kf) {
 
 // Merge NS scores (log2 domain, -inf = not attended) and their V fragments
 // into (m, l, acc): one max, one rescale, NS exponentials.
-template <typename T, int NCH, int NS>
+// DROP: the V fragment of a step t > 0 that is not ok counts as zeros (its
+// weight is 0, but 0 times an infinity is NaN); step 0 is ok.
+template <typename T, int NCH, int NS, bool DROP = false>
 __device__ __forceinline__ void fold_scores(const float* s, const Vec16 (*vf)[NCH], float& m, float& l,
-                                            float* acc) {
+                                            float* acc, const bool* ok = nullptr) {
     // (a maximum that a NaN passes through: fmaxf would drop a chunk of nothing
     // but NaN scores as one without keys)
     float cm = s[0];
@@ -204,7 +206,14 @@ __device__ __forceinline__ void fold_scores(const float* s, const Vec16 (*vf)[NC
         const float pt = fast_exp2(s[t] - m_new);  // exp2(-inf) = 0 for skipped steps
         l += pt;
 #pragma unroll
-        for (int i = 0; i < NCH; ++i) axpy8<T>(acc + 8 * i, pt, vf[t][i]);
+        for (int i = 0; i < NCH; ++i) {
+            Vec16 v = vf[t][i];
+            if (DROP && t > 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v.w[e] = ok[t] ? v.w[e] : 0u;
+            }
+            axpy8<T>(acc + 8 * i, pt, v);
+        }
     }
     m = m_new;
 }
@@ -336,6 +345,22 @@ struct Walk4 {
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+    }
+
+    // Zero the V rows of the chunk's steps without a key: those steps have
+    // weight 0, and 0 times the own row's infinity would be NaN.  (A row of
+    // zeros to read in its place is one more cache miss: 1-3% of a small call.)
+    __device__ __forceinline__ void drop_invalid() {
+        bool all = true;
+#pragma unroll
+        for (int t = 0; t < CH; ++t) all &= val[t];
+        if (__all(all)) return;
+#pragma unroll
+        for (int t = 0; t < CH; ++t)
+#pragma unroll
+            for (int i = 0; i < NCH; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vf[t][i].w[e] = val[t] ? vf[t][i].w[e] : 0u;
     }
 
     // Fold the issued chunk into one query's (m, l, acc).

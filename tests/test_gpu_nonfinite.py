@@ -135,3 +135,47 @@ def test_nan_split_reaches_its_heads(N, Hq, Hkv, D, dtype):
     assert torch.equal(torch.isnan(lse2), hit)
     assert torch.equal(torch.isnan(O2).all(-1), hit) and torch.equal(torch.isnan(O2).any(-1), hit)
     assert torch.equal(O2[~hit], O[~hit]) and torch.equal(lse2[~hit], lse[~hit])
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,D,md,walk", [
+    ([2048, 30], 32, 8, 128, 6, "heap"),   # group kernel, 4 heads per slot
+    ([2048, 30], 32, 8, 128, 6, "parents"),
+    ([2100, 30], 32, 8, 64, 6, "heap"),
+    ([2100, 30], 32, 16, 64, 1, "parents"),  # 2 heads; a walk that ends before its chunk
+    ([60], 16, 4, 128, 6, "prefix"),  # one wave per query: lane groups without a first or a second step
+    ([60], 16, 4, 64, 3, "prefix"),
+    ([60], 16, 4, 32, 3, "prefix"),
+    ([300], 8, 2, 128, 40, "prefix"),
+])
+def test_infinite_value_of_an_attended_node(lens, Hq, Hkv, D, md, walk):
+    """Where a wave holds walks of several lengths: an infinity in one element of
+    a leaf's, an inner node's and a root's V row comes out as that infinity in that element of exactly the queries that attend
+    the node (their weights are far above 0), and changes nothing else."""
+    from qattention_amd import _lib, ragged_attn as ra
+    b, L = 4, 300
+    Q, K, V, cu = make_inputs(lens, Hq, D, 9300 + D + Hkv, Hkv=Hkv)
+    par = np.concatenate([np.maximum(np.arange(n) - 1, 0) // b for n in lens]).astype(np.int32)
+    g = torch.Generator().manual_seed(9301)
+    Kp, Vp = (torch.randn(len(lens), L, Hkv, D, generator=g).half().to(DEV) for _ in range(2))
+    V2 = V.clone()
+    nodes = [lens[0] - 1, 6, 0][:Hkv]
+    for h, node in enumerate(nodes):
+        V2[node, h, 5 + h] = float("inf") if h != 1 else float("-inf")
+
+    def call(v):
+        q, k, v, pd = Q.to(DEV), K.to(DEV), v.to(DEV), torch.from_numpy(par).to(DEV)
+        if walk == "heap":
+            return ra._tree_forward(q, k, v, cu, b, md, max(lens), True, _lib.ALGO_GATHER)
+        if walk == "parents":
+            return ra.ragged_attention_with_parents(q, k, v, cu, pd, md, max(lens))
+        return ra.ragged_attention_prefix(q, k, v, cu.to(DEV), Kp, Vp, b, md, max_seqlen=max(lens), return_lse=True,
+                                          num_splits=3, parents=pd)
+
+    say("inf value", walk, lens, Hq, Hkv, D, md)
+    (O, lse), (O2, lse2) = call(V), call(V2)
+    r = Hq // Hkv
+    want = O.clone()
+    for h, node in enumerate(nodes):
+        hit = _attends(cu, b, md, None, node).to(DEV)
+        want[hit, h * r:(h + 1) * r, 5 + h] = V2[node, h, 5 + h].to(DEV)
+    assert torch.equal(O2, want) and torch.equal(lse2, lse)
