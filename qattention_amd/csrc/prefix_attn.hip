@@ -220,8 +220,9 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     const uint32_t vrow = (uint32_t)(wave * NI * RPI + lane / DV) * (uint32_t)vst;
     // First row of block i.  The last block of a range that is no multiple of
     // 64 keys starts early (its first keys, also in the block before, are
-    // masked), and a block past the end repeats it: every load of the key
-    // loop is of 64 whole rows, without a bound to clamp to.
+    // masked and their V rows cleared), and a block past the end repeats it:
+    // every load of the key loop is of 64 whole rows, without a bound to clamp
+    // to.
     auto block_row = [&](int i) { return min(k_lo + i * kBN, k_hi - kBN); };
     // a whole block at once, before the loop; block 0 may be the only one and
     // shorter than 64 rows: rows past the last repeat it
@@ -429,6 +430,17 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     // 10240-token prefix, 85 nodes x 4 sequences x 32 / 8 heads, fp16: 84.9 ->
     // 80.7 us; 4096 shared tokens, 672 x 8 x 32: 416 -> 397; 2048 tokens, 4681 x
     // 16 x 32: 2.81 -> 2.75 ms. ----
+    // The keys that the last block shares with the one before have weight 0
+    // there, and 0 times an infinity is NaN: clear their V rows (every thread
+    // of the workgroup, once the block has landed).
+    auto drop_shared = [&](int buf) {
+        const int shared = nb > 1 ? k_lo + (nb - 1) * kBN - block_row(nb - 1) : 0;
+        if (shared > 0) {
+            for (int i = tid; i < shared * DV; i += kPrefixThreads)
+                st16(Vb0 + buf * BLK + 8 * i, Vec16{{0u, 0u, 0u, 0u}});
+            publish(W0{});
+        }
+    };
     issue(kbase, kst, krow, 0, Kb0);
     issue(vbase, vst, vrow, 0, Vb0);
     if (nb > 1) {
@@ -486,6 +498,7 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
         };
         auto last = [&](auto par, f16v_t (&sc)[2]) {
             publish(W0{});  // the last V block
+            drop_shared(decltype(par)::value);
 #pragma unroll
             for (int i = 0; i < FV; ++i) va[i] = fetch_v(par, i);
 #pragma unroll
@@ -549,6 +562,7 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
             publish(W2{});
         }
         publish(W0{});
+        drop_shared((nb - 1) & 1);
     }
     __syncthreads();  // the LDS is reused by the fused epilogue
 

@@ -179,3 +179,35 @@ def test_infinite_value_of_an_attended_node(lens, Hq, Hkv, D, md, walk):
         hit = _attends(cu, b, md, None, node).to(DEV)
         want[hit, h * r:(h + 1) * r, 5 + h] = V2[node, h, 5 + h].to(DEV)
     assert torch.equal(O2, want) and torch.equal(lse2, lse)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("L,ns", [(65, 1), (127, 1), (129, 1), (200, 1), (255, 1), (193, 2), (255, 2), (500, 3)])
+def test_infinite_prefix_value_near_the_end(L, ns, D, dtype):
+    """The last key block of a prefix that is no multiple of 64 keys starts early;
+    an infinite value among the keys it shares with the block before (L - 64 is
+    always one) and of the last key comes out as that infinity, in its element
+    alone.  Small queries: no weight is near 0.  128-row tiles, the last one with
+    waves that hold no rows."""
+    from qattention_amd import ragged_attn as ra
+    B, N, b, md, Hq, Hkv = 8, 121, 3, 4, 32, 8
+    Q, K, V, cu = make_inputs([N] * B, Hq, D, 9400 + D + L, dtype=dtype, Hkv=Hkv)
+    Q = Q * 0.125
+    g = torch.Generator().manual_seed(9401)
+    Kp, Vp = (torch.randn(B, L, Hkv, D, generator=g).to(dtype) for _ in range(2))
+    call = lambda vp: ra.ragged_attention_prefix(  # noqa: E731
+        *(x.to(DEV) for x in (Q, K, V, cu, Kp, vp)), b, md, max_seqlen=N, return_lse=True, num_splits=ns)
+    say("inf prefix value", L, ns, D, dtype)
+    O, lse = call(Vp)
+    Vp2 = Vp.clone()
+    Vp2[:, L - 64, 0, 3] = float("inf")
+    Vp2[:, L - 64, 1, 4] = float("-inf")
+    Vp2[:, L - 1, 2, 5] = float("inf")
+    O2, lse2 = call(Vp2)
+    want = O.clone()
+    r = Hq // Hkv
+    want[:, :r, 3] = float("inf")
+    want[:, r:2 * r, 4] = float("-inf")
+    want[:, 2 * r:3 * r, 5] = float("inf")
+    assert torch.equal(O2, want) and torch.equal(lse2, lse)
