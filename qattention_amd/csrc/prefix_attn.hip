@@ -278,15 +278,16 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
             kad[i >> 1] + 2 * (decltype(buf)::value * BLK + 32 * D * (i & 1)));
         return Vec16{{x[0], x[1], x[2], x[3]}};
     };
-    auto fetch_v = [&](auto buf, int i) {
+    auto fetch_v_at = [&](uint32_t buf_off, int i) {
         typedef short v4s __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) v4s* lds_v4s;
-        const uint32_t off = 2 * ((2 + decltype(buf)::value) * BLK + 16 * D * (i / DT));
+        const uint32_t off = buf_off + 2 * 16 * D * (i / DT);
         const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(vxa[i % DT] + off));
         const v4s y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(vya[i % DT] + off));
         const uint2 x2 = __builtin_bit_cast(uint2, x), y2 = __builtin_bit_cast(uint2, y);
         return Vec16{{x2.x, x2.y, y2.x, y2.y}};
     };
+    auto fetch_v = [&](auto buf, int i) { return fetch_v_at(2 * (2 + decltype(buf)::value) * BLK, i); };
 
     // Online softmax (the lane's query; element r of S tile t is key 32 t +
     // 8 (r / 4) + 4 hl + r % 4 of the block).  The running max is kept on raw
@@ -319,14 +320,14 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     // -inf for the keys of a block (first row kb) outside [lo, k_hi)
     auto mask_block = [&](int kb, int lo, f16v_t (&s)[2]) {
         if (__builtin_expect(kb < lo || kb + kBN > k_hi, 0)) {
-            int k0 = kb + 4 * hl;
+            uint32_t k0 = (uint32_t)(kb - lo + 4 * hl);
             asm volatile("" : "+v"(k0));  // (32 key numbers held across the loop would spill)
+            const uint32_t keys = (uint32_t)(k_hi - lo);
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int key = k0 + 32 * t + 8 * (r >> 2) + (r & 3);
-                    if (key < lo || key >= k_hi) s[t][r] = -INFINITY;
+                    if (k0 + 32 * t + 8 * (r >> 2) + (r & 3) >= keys) s[t][r] = -INFINITY;  // (below lo: wrapped)
                 }
         }
     };
@@ -496,23 +497,6 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
             move_ref(mb);
             fence();
         };
-        auto last = [&](auto par, f16v_t (&sc)[2]) {
-            publish(W0{});  // the last V block
-            drop_shared(decltype(par)::value);
-#pragma unroll
-            for (int i = 0; i < FV; ++i) va[i] = fetch_v(par, i);
-#pragma unroll
-            for (int n = 0; n < 32; ++n) {
-                stage(sc, n, 0);
-                stage(sc, n, 1);
-                stage(sc, n, 2);
-            }
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                oacc[i % DT] = mma32<T>(va[i % FV], pf[i / DT], oacc[i % DT]);
-                if (i + FV < NP) va[i % FV] = fetch_v(par, i + FV);
-            }
-        };
         f16v_t sA[2], sB[2];
         zero(sA);
 #pragma unroll
@@ -540,9 +524,29 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
         }
         if (j + 1 < nb) {
             iter(j, B0{}, sA, sB);
-            last(B1{}, sB);
-        } else {
-            last(B0{}, sA);
+            sA[0] = sB[0];
+            sA[1] = sB[1];
+        }
+        // ---- the last block, in one copy for both buffers (a copy for each
+        // took D = 128 past 256 VGPRs) ----
+        const uint32_t vbuf = 2 * (2 + ((nb - 1) & 1)) * BLK;
+        publish(W0{});
+        drop_shared((nb - 1) & 1);
+#pragma unroll
+        for (int i = 0; i < FV; ++i) va[i] = fetch_v_at(vbuf, i);
+        // its weights, those of each 16-key step beside the products of the one before
+#pragma unroll
+        for (int i = -DT; i < NP; ++i) {
+#pragma unroll
+            for (int n = 0; n < 32; ++n) {
+                if (n * DT / 8 != i + DT) continue;
+                stage(sA, n, 0);
+                stage(sA, n, 1);
+                stage(sA, n, 2);
+            }
+            if (i < 0) continue;
+            oacc[i % DT] = mma32<T>(va[i % FV], pf[i / DT], oacc[i % DT]);
+            if (i + FV < NP) va[i % FV] = fetch_v_at(vbuf, i + FV);
         }
         __builtin_amdgcn_s_setprio(0);
         l_run = ps0 + ps1;
