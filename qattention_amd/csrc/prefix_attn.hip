@@ -302,7 +302,10 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     // the reference's FA2 loop does; fp16 (11 bits) keeps the lazy reference.
     const float csc = p.scale_log2;
     constexpr float kLazy = T::kCode == QATTN_DTYPE_BF16 ? 0.f : 8.f;
-    float mc = 0.f, ps0 = 0.f, ps1 = 0.f;  // m_run csc; the lane's sum of weights, in two parts
+    // m_run csc; the sum of one block's weights, in two parts (summed by block,
+    // then over the blocks: one running sum of every weight doubled the LSE's
+    // error, 2.0e-6 -> 5.5e-6 over 200000 keys)
+    float mc = 0.f, ps0 = 0.f, ps1 = 0.f;
     auto move_ref = [&](float mb) {
         mb = xor32_max(mb);
         const bool move = (mb - m_run) * csc > kLazy;  // always true on the first block
@@ -311,8 +314,7 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
             const float alpha = move ? fast_exp2((m_run - m_new) * csc) : 1.f;  // m_run = -inf: 0
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
-            ps0 *= alpha;
-            ps1 *= alpha;
+            l_run *= alpha;
             m_run = m_new;
         }
         mc = m_run * csc;
@@ -345,10 +347,10 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
         s[n >> 4][n & 15] = x;
         if (q == 2) {
             if (n & 1) {
-                ps1 += x;
+                ps1 = n == 1 ? x : ps1 + x;
                 pf[n >> 3].w[(n & 7) >> 1] = MfmaOps<T>::pack2(s[n >> 4][(n & 15) - 1], x);
             } else {
-                ps0 += x;
+                ps0 = n == 0 ? x : ps0 + x;
             }
         }
     };
@@ -494,6 +496,7 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
                         mb = fmaxf(fmaxf(mb, sn[e >> 3][2 * (e & 7)]), sn[e >> 3][2 * (e & 7) + 1]);
                 fence();
             }
+            l_run += ps0 + ps1;
             move_ref(mb);
             fence();
         };
@@ -549,7 +552,7 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
             if (i + FV < NP) va[i % FV] = fetch_v_at(vbuf, i + FV);
         }
         __builtin_amdgcn_s_setprio(0);
-        l_run = ps0 + ps1;
+        l_run += ps0 + ps1;
     } else {
         // a wave past the tile's rows only stages its part of the blocks (672
         // rows per kv head leave 3 of 24 waves without any: 408 -> 397 us)

@@ -44,3 +44,33 @@ def test_blocks_per_range(blocks, D, dtype, splits):
         assert (np.abs(o - o_ref) <= bound).all(), (last, N, np.abs(o - o_ref).max())
         err = np.abs(lse.double().cpu().numpy() - lse_ref).max()
         assert err <= (1e-4 if dtype == torch.float16 else 1e-3), (last, N, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_small_weights_after_a_large_one(D, dtype):
+    """One key of weight 1 and 2^17 of weight 2^-25: added one by one to a sum
+    above 1 each would round away (a quarter of the 2^-8 in all, those of one
+    lane's partial sum: 1e-3 of the LSE); added block by block 16 of them are 4
+    ulps.  Both weights are within 1e-3 of those powers, so a block's 4 ulps
+    round to 4 and at most 2^-10 of 2^-8 is lost: 4e-6, and 4e-6 for the fp32
+    sums and the logarithm."""
+    from qattention_amd import ragged_attn as ra
+    L = 1 + 2 ** 17
+    step = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    mant = 1.0 + step * np.arange(0, int(1 / step), max(1, int(1 / step) // 64))
+    c = 1.0 + step * np.arange(int(1 / step))
+    s = mant[:, None] * c[None, :] * 64 / np.sqrt(D) * np.log2(np.e)  # (both times 8)
+    pow2 = 2.0 ** np.round(np.log2(25 / s))
+    i, j = np.unravel_index(np.abs(s * pow2 - 25).argmin(), s.shape)
+    Q = torch.zeros(1, 1, D)
+    Q[0, 0, 0] = mant[i] * 8 * pow2[i, j]
+    K = torch.zeros(L, 1, D)
+    K[0, 0, 0] = c[j] * 8
+    Q, K = Q.to(dtype).to(DEV), K.to(dtype).to(DEV)
+    score = float(Q[0, 0, 0]) * float(K[0, 0, 0]) / np.sqrt(D)
+    assert abs(score * np.log2(np.e) - 25) < 1e-3, score
+    print("small weights", D, dtype, score, flush=True)
+    _, lse = ra.prefix_attention(Q, K, torch.zeros_like(K), num_splits=1)
+    want = score + np.log1p((L - 1) * np.exp(-score))
+    assert abs(float(lse[0, 0]) - want) <= 8e-6, (float(lse[0, 0]), want)
