@@ -203,6 +203,13 @@ int qattn_ancestors(const int32_t *cu_seqlens, const int32_t *parents, int32_t b
 int qattn_debug_walk(int32_t *out);
 
 /*
+ * Name of the last kernel that a call of this thread launched ("" before the
+ * first; the group kernel's with its heads or lanes per slot), for tests of
+ * the rules that choose one.
+ */
+const char *qattn_debug_last_kernel(void);
+
+/*
  * Tree-verify attention with a prefix KV cache that every tree query attends
  * in full, plus its own ancestors among the tree tokens.
  *

@@ -41,6 +41,7 @@ SIGNATURES = {
     "qattn_init": (C.c_int, []),
     "qattn_sched_info": (C.c_int, [_i64p]),
     "qattn_debug_walk": (C.c_int, [_p]),
+    "qattn_debug_last_kernel": (C.c_char_p, []),
     "qattn_tree_fwd": (C.c_int, [
         _p, _i64p, _p, _i64p, _p, _i64p, _p, _i64p, _p, _i64p,
         _p, _i32, _i32, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _p]),
@@ -125,6 +126,11 @@ def debug_walk(table):
         yield table
     finally:
         lib().qattn_debug_walk(None)
+
+
+def last_kernel() -> str:
+    """Name of the last kernel that a call of this thread launched."""
+    return lib().qattn_debug_last_kernel().decode()
 
 
 def sched_info(device=None) -> dict:

@@ -55,6 +55,8 @@ void clear_error() { g_err[0] = 0; }
 
 // The calling thread's walk-export table (qattn_debug_walk), or null.
 static thread_local int32_t* g_dbg_walk = nullptr;
+// The calling thread's last launch (qattn_debug_last_kernel).
+static thread_local const char* g_last_kernel = "";
 
 // ---------------------------------------------------------------------------
 // Gather kernel: 4 lanes per (token, q head), 64 pairs per workgroup with the
@@ -453,6 +455,7 @@ int launch_status(const char* what) {
         set_error("%s: %s", what, hipGetErrorString(e));
         return QATTN_ERR_HIP;
     }
+    g_last_kernel = what;
     return QATTN_OK;
 }
 
@@ -617,7 +620,8 @@ static int launch_group_gs(const TreeParams& p, hipStream_t st) {
     else
         hipLaunchKernelGGL((tree_group_kernel<T, D, WALK, LAYOUT, GS, LPR>), dim3((unsigned)blocks), dim3(kThreads), 0,
                            st, p, hg, pg);
-    return launch_status("tree_group_kernel");
+    return launch_status(GS > 1 ? (GS == 4 ? "tree_group_kernel, 4 heads" : "tree_group_kernel, 2 heads")
+                                : (LPR == 16 ? "tree_group_kernel, 16 lanes" : "tree_group_kernel, 8 lanes"));
 }
 
 // q heads per slot and lanes per row of the group kernel for a call; gs 0: the
@@ -867,6 +871,8 @@ int qattn_debug_walk(int32_t* out) {
     g_dbg_walk = out;
     return QATTN_OK;
 }
+
+const char* qattn_debug_last_kernel(void) { return g_last_kernel; }
 
 int qattn_tree_fwd(const void* q, const int64_t q_stride[3], const void* k, const int64_t k_stride[3],
                    const void* v, const int64_t v_stride[3], void* o, const int64_t o_stride[3], float* lse,

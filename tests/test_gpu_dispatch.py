@@ -1,0 +1,78 @@
+"""Which kernel a call gets, at each limit of the dispatch rules and one past it.
+
+The outputs of every case are checked against the fp64 oracle too (fp16 2e-3,
+half an ulp of |o| in [4, 8); bf16 2^-7 max(1, |o|) + 1e-3, one rounding of O)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import make_inputs, oracle_tree
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+GATHER, STREAM, MERGE = "tree_gather_kernel", "tree_stream_kernel", "tree_merge_kernel"
+H2, H4 = "tree_group_kernel, 2 heads", "tree_group_kernel, 4 heads"
+L8, L16 = "tree_group_kernel, 8 lanes", "tree_group_kernel, 16 lanes"
+
+
+def _parents(lens, b):
+    return np.concatenate([np.maximum(np.arange(n) - 1, 0) // b for n in lens]).astype(np.int32)
+
+
+def _check(O, ref, dtype, what):
+    bound = 2e-3 if dtype == torch.float16 else 2.0 ** -7 * np.maximum(1.0, np.abs(ref)) + 1e-3
+    assert (np.abs(O.double().cpu().numpy() - ref) <= bound).all(), what
+
+
+def _walk(walk, lens, b, md, Hq, Hkv, D, algo):
+    from qattention_amd import _lib, ragged_attn as ra
+    Q, K, V, cu = make_inputs(lens, Hq, D, 9500 + md + D, Hkv=Hkv)
+    q, k, v = Q.to(DEV), K.to(DEV), V.to(DEV)
+    print("walk", walk, lens, b, md, Hq, Hkv, D, flush=True)
+    par = None
+    if walk == "heap":
+        O, _ = ra._tree_forward(q, k, v, cu, b, md, max(lens), False, algo)
+    elif walk == "parents":
+        par = _parents(lens, b)
+        O, _ = ra.ragged_attention_with_parents(q, k, v, cu, torch.from_numpy(par).to(DEV), md, max(lens))
+    else:
+        Kc, Vc, pt = ra.build_paged_kv(list(k.split(lens)), list(v.split(lens)), 16)
+        O, _ = ra._paged_forward(q, Kc, Vc, pt.to(DEV), cu, b, md, max(lens), False, algo)
+    name = _lib.last_kernel()
+    _check(O, oracle_tree(Q, K, V, cu, b, md, parents=par)[0], torch.float16, walk)
+    return name
+
+
+@pytest.mark.parametrize("lens,b,md,Hq,Hkv,D,want", [
+    # 4 heads per slot from 2048 waves on (4 lanes per slot at D = 32, else 8), 2 from 4096
+    ([2048], 4, 5, 32, 8, 128, H4),
+    ([2047], 4, 5, 32, 8, 128, GATHER),
+    ([4096], 4, 6, 32, 8, 32, H4),
+    ([4095], 4, 6, 32, 8, 32, GATHER),
+    ([4096], 4, 6, 16, 8, 64, H2),
+    ([4095], 4, 6, 16, 8, 64, GATHER),
+    # one head, 16 lanes at D = 128: 8192 queries
+    ([256], 2, 8, 32, 8, 128, L16),
+    ([257], 2, 8, 32, 8, 128, GATHER),
+    # 8 lanes at D = 128: up to 65536 queries of at most 4 steps
+    ([2048], 28, 3, 32, 32, 128, L8),
+    ([2049], 28, 3, 32, 32, 128, GATHER),
+    ([2048], 2, 4, 32, 32, 128, GATHER),
+])
+@pytest.mark.parametrize("walk", ["heap", "parents", "paged"])
+def test_walk_kernel(lens, b, md, Hq, Hkv, D, want, walk):
+    from qattention_amd import _lib
+    assert _walk(walk, lens, b, md, Hq, Hkv, D, _lib.ALGO_GATHER) == want
+
+
+@pytest.mark.parametrize("B,N,b,md,Hq,Hkv,D,want", [
+    (1, 672, 28, 2, 32, 32, 128, L8),
+    (4, 1365, 4, 5, 32, 32, 128, STREAM),
+    (24, 341, 4, 4, 32, 8, 64, H4),
+    (8, 1023, 2, 9, 32, 8, 128, STREAM),
+])
+def test_auto_choice(B, N, b, md, Hq, Hkv, D, want):
+    from qattention_amd import _lib
+    assert _walk("heap", [N] * B, b, md, Hq, Hkv, D, _lib.ALGO_AUTO) == want
