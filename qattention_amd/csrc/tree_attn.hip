@@ -64,10 +64,16 @@ static thread_local const char* g_last_kernel = "";
 // ---------------------------------------------------------------------------
 // DBG: the walk-export instantiation (qattn_debug_walk): every query's walk
 // steps are also written to p.dbg_walk.
-template <typename T, int D, int WALK, int LAYOUT, bool LSE, bool PSTATE, bool BATCH, bool DBG = false>
+// TPB: threads per workgroup.  A split merge that would occupy under half
+// the CUs takes one wave per workgroup instead, so four times the CUs share
+// its loads (each CU's vector memory path, not latency, bounds such a launch:
+// 4 x 60 nodes x 32 heads over 2048 tokens, D = 64 19.5 -> 19.2 us, 500 nodes x
+// 8 heads 14.4 -> 13.8).
+template <typename T, int D, int WALK, int LAYOUT, bool LSE, bool PSTATE, bool BATCH, bool DBG = false,
+          int TPB = kThreads>
 __global__ __launch_bounds__(kThreads) void tree_gather_kernel(TreeParams p) {
     constexpr int NCH = D / 32;
-    constexpr int SLOTS = kThreads / 4;
+    constexpr int SLOTS = TPB / 4;
     const int j = threadIdx.x & 3;
     // Without split states: XCD-contiguous block order.  The dispatcher
     // places block i on XCD i % 8, so XCD x takes the x-th eighth of the
@@ -563,6 +569,25 @@ static bool make_subtree_plan(int b, int64_t n, int max_depth, int rcap, int nca
     return rows <= rcap;
 }
 
+// Queries up to which a split merge takes one wave each (tree_merge_kernel).
+// The fewer bytes a state and a row hold, the sooner a whole wave per query
+// costs more issue slots than the shorter chain of loads saves; and one small
+// tree finds its states in the L2 that wrote them.  Whole steps over 2048
+// tokens, us, gather / merge kernel, fp16 unless noted:
+//  D = 128: one tree of 16-250 nodes x 32 heads 1.2-1.3 times as fast (128 nodes
+//    20.0 / 16.1, 250 29.5 / 25.0); 500 x 8 heads 19.6 / 18.5, 2 x 60 x 32 20.5 /
+//    20.4, 4 x 60 x 32 28.0 / 28.8, 1000 x 8 29.4 / 30.1
+//  D = 64: one tree of 128 x 32 13.9 / 12.5, 250 x 32 19.8 / 18.7, bf16 24.1 /
+//    19.9; 300 x 8 12.6 / 12.1, 2 x 60 x 32 13.8 / 14.6, 4 x 60 x 32 19.2 / 22.6
+//  D = 32: 1024 queries 9.2 / 9.2, 2400 10.6 / 11.1, 8000 13.2 / 16.5; bf16 3072
+//    12.0 / 11.2, 4000 12.3 / 13.1
+template <typename T, int D>
+static int64_t merge_limit(const TreeParams& p) {
+    if (D == 32) return kPartHalf<T> ? 1024 : 3072;
+    if (p.B == 1 && p.max_seqlen <= kMergeParents) return 8192;
+    return D == 64 ? 3072 : 6144;
+}
+
 template <typename T, int D, int WALK, int LAYOUT, bool LSE, bool PSTATE, bool BATCH = false, bool DBG = false>
 static int launch_gather(const TreeParams& p, hipStream_t st) {
     constexpr int SLOTS = kThreads / 4;  // 4 lanes per (token, q head)
@@ -573,13 +598,17 @@ static int launch_gather(const TreeParams& p, hipStream_t st) {
         return QATTN_ERR_ARG;
     }
     if constexpr (PSTATE && LAYOUT == KV_PACKED) {
-        // one wave per query below 8 waves per SIMD (8 x 60 queries x 32 heads:
-        // 41.6 us by the gather kernel, 44.9 by this one; 4 x 60: 43.2 and 40.9)
-        if (slots < 8192) {
+        if (slots <= merge_limit<T, D>(p)) {
             constexpr int WAVES = kThreads / 64;
             hipLaunchKernelGGL((tree_merge_kernel<T, D, WALK, BATCH, DBG>),
                                dim3((unsigned)((slots + WAVES - 1) / WAVES)), dim3(kThreads), 0, st, p);
             return launch_status("tree_merge_kernel");
+        }
+        if (blocks < 128) {
+            constexpr int S1 = 64 / 4;
+            hipLaunchKernelGGL((tree_gather_kernel<T, D, WALK, LAYOUT, LSE, PSTATE, BATCH, DBG, 64>),
+                               dim3((unsigned)((slots + S1 - 1) / S1)), dim3(64), 0, st, p);
+            return launch_status("tree_gather_kernel");
         }
     }
     hipLaunchKernelGGL((tree_gather_kernel<T, D, WALK, LAYOUT, LSE, PSTATE, BATCH, DBG>), dim3((unsigned)blocks),

@@ -76,3 +76,32 @@ def test_walk_kernel(lens, b, md, Hq, Hkv, D, want, walk):
 def test_auto_choice(B, N, b, md, Hq, Hkv, D, want):
     from qattention_amd import _lib
     assert _walk("heap", [N] * B, b, md, Hq, Hkv, D, _lib.ALGO_AUTO) == want
+
+
+@pytest.mark.parametrize("B,N,Hq,Hkv,D,dtype,want", [
+    # one tree of up to 256 nodes: 8192 queries, else 6144 at D = 128 and 3072 at 64
+    (1, 256, 32, 8, 128, torch.float16, MERGE),
+    (1, 257, 32, 8, 128, torch.float16, GATHER),
+    (2, 96, 32, 8, 128, torch.float16, MERGE),
+    (2, 97, 32, 8, 128, torch.bfloat16, GATHER),
+    (1, 256, 32, 8, 64, torch.bfloat16, MERGE),
+    (2, 48, 32, 8, 64, torch.float16, MERGE),
+    (2, 49, 32, 8, 64, torch.float16, GATHER),
+    # D = 32: 1024 fp16, 3072 bf16
+    (1, 32, 32, 8, 32, torch.float16, MERGE),
+    (1, 33, 32, 8, 32, torch.float16, GATHER),
+    (1, 96, 32, 8, 32, torch.bfloat16, MERGE),
+    (1, 97, 32, 8, 32, torch.bfloat16, GATHER),
+])
+def test_split_merge_kernel(B, N, Hq, Hkv, D, dtype, want):
+    from qattention_amd import _lib, ragged_attn as ra
+    b, md, L = 3, 5, 300
+    Q, K, V, cu = make_inputs([N] * B, Hq, D, 9600 + N + D, dtype=dtype, Hkv=Hkv)
+    g = torch.Generator().manual_seed(9601)
+    Kp, Vp = (torch.randn(B, L, Hkv, D, generator=g).to(dtype) for _ in range(2))
+    print("merge", B, N, Hq, Hkv, D, dtype, flush=True)
+    for par in (None, _parents([N] * B, b)):
+        O = ra.ragged_attention_prefix(*(x.to(DEV) for x in (Q, K, V, cu, Kp, Vp)), b, md, max_seqlen=N, num_splits=3,
+                                       parents=None if par is None else torch.from_numpy(par).to(DEV))
+        assert _lib.last_kernel() == want
+        _check(O, oracle_tree(Q, K, V, cu, b, md, parents=par, Kp=Kp, Vp=Vp)[0], dtype, (B, N, D))
