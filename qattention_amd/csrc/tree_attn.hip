@@ -665,13 +665,20 @@ struct GroupPlan {
 // against 12.1 us, 2000 15.8 against 17.2, 8000 41.8 against 49.3; D = 64: 2000
 // waves equal, 3000 12.2 against 13.9; 16/8 heads: 3000 13.5 against 13.0, 4000
 // 16.0 against 17.4).  At the other end the gather kernel's 4 lanes per query
-// leave the chip idle: one 16-byte chunk per lane (D / 8 lanes) ran 60 nodes
-// b=2, 32 heads, D = 128 in 4.75 against 5.76 us, 250 nodes in 5.42 against 6.11,
-// 500 nodes with 32/8 heads in 6.15 against 6.27, and 8 lanes one 672-node b=28
-// tree (3 steps) in 7.5 against 8.8 us, three of them in 16.8 against 17.9, but
-// 1000 nodes b=3 (7 steps) in 12.8 against 12.5.  Packed layouts (cu) without
-// split states only.  steps: walk steps per query, at most.
-static GroupPlan group_plan(const TreeParams& p, int head_dim, int steps, bool pstate) {
+// leave the chip idle.  One 16-byte chunk per lane at D = 128 (16 lanes): 64 to
+// 4096 queries b=2 1.25 times as fast, 8192 with explicit parents 4.5 against
+// 5.7 us, paged 4.7 against 5.0; ungrouped heads 12288 5.5 against 6.4, b=8 3.9
+// against 4.1, but 14400 b=8 5.0 against 4.8 and paged 9600 5.4 against 5.1.
+// 8 lanes ran one 672-node b=28 tree (3 steps) in 7.5 against 8.8 us, three
+// of them in 16.8 against 17.9, but 1000 nodes b=3 (7 steps) in 12.8 against
+// 12.5.  At D = 64 (8 lanes) a round of loads covers 2 steps against 4, so it
+// pays where it takes less than twice the rounds (5 steps 3.37 against 3.62
+// us, paged 4.00 against 4.14; 4 steps 3.02 against 2.91, paged 3.44 against
+// 3.13; 8 steps 3.97 against 3.72) and for the dependent loads of explicit
+// parents (7 steps 3.95 against 4.09), up to 8192 queries (12288: 4.6 against
+// 4.3).  Packed layouts (cu) without split states only.  steps: walk steps
+// per query, at most.
+static GroupPlan group_plan(const TreeParams& p, int head_dim, int walk, int layout, int steps, bool pstate) {
     const int64_t queries = (int64_t)p.B * p.max_seqlen * p.Hq;
     if (!p.cu || pstate || queries >= (int64_t(1) << 31)) return {0, 0};
     if (p.group % 2 == 0) {
@@ -679,7 +686,12 @@ static GroupPlan group_plan(const TreeParams& p, int head_dim, int steps, bool p
         if (queries / gs * lanes / 64 >= 8192 / gs) return {gs, lanes};
     }
     if (head_dim == 32) return {0, 0};
-    if (queries <= (p.group == 1 ? 16384 : 8192)) return {1, head_dim / 8};
+    if (head_dim == 64 && queries <= 8192) {
+        // 8 lanes load 2 steps per round, the gather kernel's 4 lanes 4
+        const bool rounds = steps % 4 == 1 || steps % 4 == 2;
+        return rounds || (walk == WALK_PARENTS && steps > 4) ? GroupPlan{1, 8} : GroupPlan{0, 0};
+    }
+    if (head_dim == 128 && queries <= (p.group == 1 && layout != KV_PAGED ? 12288 : 8192)) return {1, 16};
     if (head_dim == 128 && p.group == 1 && queries <= 65536 && steps <= 4) return {1, 8};
     return {0, 0};
 }
@@ -772,7 +784,7 @@ static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bo
         // (uniform batches have no group kernel and keep the tile rule).
         const bool use = ok && (algo == QATTN_ALGO_SUBTREE ||
                                 (wgs >= (pstate ? 2048 : 512) &&
-                                 (pstate || !p.cu || subtree_pays(p, plan, D, paged, group_plan(p, D, steps, false).gs))));
+                                 (pstate || !p.cu || subtree_pays(p, plan, D, paged, group_plan(p, D, walk, layout, steps, false).gs))));
         if (algo == QATTN_ALGO_SUBTREE && !ok) {
             if (!paged_ok)
                 set_error("paged subtree kernel: page-table entries %lld (at most %d), page size %d (at most "
@@ -788,7 +800,7 @@ static int dispatch_tree(const TreeParams& p, int walk, int layout, bool lse, bo
         set_error("the subtree kernel supports the heap walk on packed or paged K/V only");
         return QATTN_ERR_ARG;
     }
-    const GroupPlan gp = group_plan(p, D, steps, pstate);
+    const GroupPlan gp = group_plan(p, D, walk, layout, steps, pstate);
     if (gp.gs) return launch_group<T, D>(p, gp, walk, layout, st);
     if (p.dbg_walk) {
         // walk export: calls over packed cu_seqlens, either dtype, with or without LSE

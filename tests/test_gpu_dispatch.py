@@ -105,3 +105,31 @@ def test_split_merge_kernel(B, N, Hq, Hkv, D, dtype, want):
                                        parents=None if par is None else torch.from_numpy(par).to(DEV))
         assert _lib.last_kernel() == want
         _check(O, oracle_tree(Q, K, V, cu, b, md, parents=par, Kp=Kp, Vp=Vp)[0], dtype, (B, N, D))
+
+
+@pytest.mark.parametrize("walk,lens,b,md,Hq,Hkv,want", [
+    # 8 lanes at D = 64, up to 8192 queries, where 2 steps a round take less than
+    # twice the rounds of 4 steps
+    ("heap", [31], 2, 9, 32, 32, L8),      # 5 steps
+    ("heap", [15, 15], 2, 3, 4, 4, GATHER),  # 4
+    ("heap", [100], 28, 9, 32, 8, GATHER),  # 3
+    ("heap", [200], 2, 9, 32, 8, GATHER),   # 8
+    ("heap", [256], 2, 9, 32, 32, L8),     # 9
+    ("heap", [257], 2, 9, 32, 32, GATHER),  # 8224 queries
+    ("paged", [200], 4, 9, 32, 32, L8),    # 5
+    ("paged", [80], 4, 9, 32, 32, GATHER),  # 4
+    # explicit parents: more than 4 steps
+    ("parents", [200], 4, 7, 32, 8, L8),
+    ("parents", [200], 4, 3, 32, 8, GATHER),
+])
+def test_walk_kernel_d64(walk, lens, b, md, Hq, Hkv, want):
+    from qattention_amd import _lib
+    assert _walk(walk, lens, b, md, Hq, Hkv, 64, _lib.ALGO_GATHER) == want
+
+
+@pytest.mark.parametrize("walk,N,want", [("heap", 384, L16), ("heap", 385, GATHER), ("parents", 384, L16),
+                                         ("parents", 385, GATHER), ("paged", 256, L16), ("paged", 257, GATHER)])
+def test_walk_kernel_ungrouped_heads(walk, N, want):
+    """16 lanes at D = 128: 12288 queries of ungrouped heads, paged 8192."""
+    from qattention_amd import _lib
+    assert _walk(walk, [N], 2, 9, 32, 32, 128, _lib.ALGO_GATHER) == want
