@@ -664,7 +664,10 @@ struct GroupPlan {
 // and 16 for GS = 2 (500-node trees b=3, 32/8 heads, D = 128: 1500 waves 13.9
 // against 12.1 us, 2000 15.8 against 17.2, 8000 41.8 against 49.3; D = 64: 2000
 // waves equal, 3000 12.2 against 13.9; 16/8 heads: 3000 13.5 against 13.0, 4000
-// 16.0 against 17.4).  At the other end the gather kernel's 4 lanes per query
+// 16.0 against 17.4), and at D = 128, where a round is one step, four times that
+// for walks of more than 32 steps (64 steps, 32/8 heads: 4000 waves 136 against
+// 125 us, 8000 equal; 16/8 heads 8000 136 against 124; 32 steps no slower from
+// 2000).  At the other end the gather kernel's 4 lanes per query
 // leave the chip idle.  One 16-byte chunk per lane at D = 128 (16 lanes): 64 to
 // 4096 queries b=2 1.25 times as fast, 8192 with explicit parents 4.5 against
 // 5.7 us, paged 4.7 against 5.0; ungrouped heads 12288 5.5 against 6.4, b=8 3.9
@@ -683,7 +686,8 @@ static GroupPlan group_plan(const TreeParams& p, int head_dim, int walk, int lay
     if (!p.cu || pstate || queries >= (int64_t(1) << 31)) return {0, 0};
     if (p.group % 2 == 0) {
         const int gs = p.group % 4 == 0 ? 4 : 2, lanes = group_lanes(head_dim);
-        if (queries / gs * lanes / 64 >= 8192 / gs) return {gs, lanes};
+        const int64_t waves = queries / gs * lanes / 64, need = 8192 / gs;
+        if (waves >= (head_dim == 128 && steps > 32 ? 4 * need : need)) return {gs, lanes};
     }
     if (head_dim == 32) return {0, 0};
     if (head_dim == 64 && queries <= 8192) {

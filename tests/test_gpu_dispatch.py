@@ -133,3 +133,11 @@ def test_walk_kernel_ungrouped_heads(walk, N, want):
     """16 lanes at D = 128: 12288 queries of ungrouped heads, paged 8192."""
     from qattention_amd import _lib
     assert _walk(walk, [N], 2, 9, 32, 32, 128, _lib.ALGO_GATHER) == want
+
+
+@pytest.mark.parametrize("N,md,want", [(2048, 31, H4), (2048, 32, GATHER), (8191, 40, GATHER), (8192, 40, H4)])
+def test_deep_walk_kernel(N, md, want):
+    """Walks of more than 32 steps at D = 128 need four times the waves."""
+    from qattention_amd import _lib
+    for walk in ("heap", "parents"):
+        assert _walk(walk, [N], 1, md, 32, 8, 128, _lib.ALGO_GATHER) == want
