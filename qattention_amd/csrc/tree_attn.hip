@@ -331,6 +331,7 @@ __global__ __launch_bounds__(kThreads) void tree_merge_kernel(TreeParams p) {
                 if (j == 0 && ok[u]) dbg[t0 + u * NG + g] = node[u];
             }
         }
+        __builtin_amdgcn_sched_barrier(0);  // every row is requested before the first wait
         if (t0 == 0) {
             fold_state(st0);
             fold_state(st1);
@@ -341,7 +342,28 @@ __global__ __launch_bounds__(kThreads) void tree_merge_kernel(TreeParams p) {
             const float d = qk4<T, 1, LPR>(&qf, &kf[u]) * p.scale_log2;
             sc[u] = ok[u] ? d : -INFINITY;
         }
-        if (ok[0]) fold_scores<T, 1, 2, true>(sc, vf, m, l, acc, ok);
+        // fold_scores without its early return (under a branch the compiler
+        // sinks the V loads behind the scores, one more round trip); a lane
+        // group without a step adds zeros
+        const float m_new = __builtin_elementwise_maximum(m, __builtin_elementwise_maximum(sc[0], sc[1]));
+        const float ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = fast_exp2(m - ref);
+        float p0 = fast_exp2(sc[0] - ref), p1 = fast_exp2(sc[1] - ref);
+        l = __builtin_fmaf(l, alpha, p0 + p1);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] *= alpha;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            // (weight 0 times an infinity in the own row would be NaN; the
+            // empty statement keeps these first uses of V behind the scores)
+            uint32_t(&w)[4] = vf[u][0].w;
+            asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(u ? p1 : p0));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = ok[u] ? w[e] : 0u;
+        }
+        axpy8<T>(acc, p0, vf[0][0]);
+        axpy8<T>(acc, p1, vf[1][0]);
+        m = m_new;
     }
     for (int s = 2 * NG + g; s < p.n_split; s += NG) fold_state(load_state(s));
     // ---- merge the groups ----

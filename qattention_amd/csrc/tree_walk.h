@@ -183,11 +183,9 @@ __device__ __forceinline__ float qk4(const Vec16* qf, const Vec16* kf) {
 
 // Merge NS scores (log2 domain, -inf = not attended) and their V fragments
 // into (m, l, acc): one max, one rescale, NS exponentials.
-// DROP: the V fragment of a step t > 0 that is not ok counts as zeros (its
-// weight is 0, but 0 times an infinity is NaN); step 0 is ok.
-template <typename T, int NCH, int NS, bool DROP = false>
+template <typename T, int NCH, int NS>
 __device__ __forceinline__ void fold_scores(const float* s, const Vec16 (*vf)[NCH], float& m, float& l,
-                                            float* acc, const bool* ok = nullptr) {
+                                            float* acc) {
     // (a maximum that a NaN passes through: fmaxf would drop a chunk of nothing
     // but NaN scores as one without keys)
     float cm = s[0];
@@ -206,14 +204,7 @@ __device__ __forceinline__ void fold_scores(const float* s, const Vec16 (*vf)[NC
         const float pt = fast_exp2(s[t] - m_new);  // exp2(-inf) = 0 for skipped steps
         l += pt;
 #pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            Vec16 v = vf[t][i];
-            if (DROP && t > 0) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v.w[e] = ok[t] ? v.w[e] : 0u;
-            }
-            axpy8<T>(acc + 8 * i, pt, v);
-        }
+        for (int i = 0; i < NCH; ++i) axpy8<T>(acc + 8 * i, pt, vf[t][i]);
     }
     m = m_new;
 }
