@@ -271,7 +271,7 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     };
     constexpr int NS = 2 * KS;  // products of S^T per block: k-step i / 2, key tile i % 2
     constexpr int NP = 4 * DT;  // products of O^T per block: 16-key step i / DT, d-tile i % DT
-    constexpr int PF = 3;       // operands read ahead of their product (4 took the split kernel past 256 VGPRs)
+    constexpr int PF = 3;       // operands read ahead of their product
     auto fetch_k = [&](auto buf, int i) {
         typedef uint32_t v4u __attribute__((ext_vector_type(4)));
         const v4u x = *(__attribute__((address_space(3))) const v4u*)(uintptr_t)(
@@ -424,12 +424,13 @@ __global__ __launch_bounds__(kPrefixThreads) __attribute__((amdgpu_waves_per_eu(
     // Waves in odd iterations run at a higher priority, which keeps the two
     // side by side (64.5 +- 3 us).
     //
-    // What bounds it: power.  The chip clocks at 1.62-1.7 GHz in this loop
-    // (2.35 with one workgroup per CU) and a wave pair takes 2770 cycles per
-    // block for 2048 cycles of matrix products; a loop of this instruction
-    // mix without dependencies or waits sustained 80% of the matrix cores at
-    // 1.6 GHz.  The previous form (products and softmax in compiler order, DMA
-    // issued at the top) took 2830-3080 cycles at 1.7-1.75 GHz.
+    // What bounds it: the matrix products at the clock that the chip's power
+    // leaves.  It runs at 1.62-1.7 GHz in this loop (2.35 with one workgroup
+    // per CU), and a wave pair takes 2770 cycles per block for 2048 cycles of
+    // products: 1287 TFLOP/s at 1.66 GHz, 74% of the matrix cores.  (Over a
+    // whole call of 16 x 4681 nodes: 54% at 1.62 GHz, counters.)  The form
+    // before (products and softmax in compiler order, DMA issued at the top)
+    // took 2830-3080 cycles at 1.7-1.75 GHz.
     // 10240-token prefix, 85 nodes x 4 sequences x 32 / 8 heads, fp16: 84.9 ->
     // 80.7 us; 4096 shared tokens, 672 x 8 x 32: 416 -> 397; 2048 tokens, 4681 x
     // 16 x 32: 2.81 -> 2.75 ms. ----
@@ -1245,8 +1246,9 @@ static int prefix_splits(int64_t ups, int L, int num_splits, int& blocks_per_spl
         // few query rows (one decode step of a small tree) that traffic and the
         // per-split overheads outgrow the split's own work.  Keep at least an
         // eighth of the blocks, within 2..8, per split (one EAGLE-3 step over
-        // a 2048-token cache runs 17.2 us per call with 8 splits, 18.8 with 4,
-        // 21.5 with 16).
+        // a 2048-token cache, prefix and merge kernel: 13.8 us with 8 splits,
+        // 16.4 with 4, 15.4 with 12, 16.3 with 16; over 8192 tokens 26.8 with 8,
+        // 27.7 with 12, 29.9 with 16; over 512 11.4 from 8 on).
         const int bps_min = std::min(8, std::max(2, blocks / 8));
         s = std::min(s, std::max(1, blocks / bps_min));
     }

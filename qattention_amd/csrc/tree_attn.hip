@@ -211,7 +211,8 @@ __global__ __launch_bounds__(kThreads) void tree_group_kernel(TreeParams p, Divi
 // K/V rows are one round trip each.  One step of a 60-node depth-7 draft tree
 // over 2048 tokens, 32/8 heads, D = 128, 8 splits, both kernels: 4 lanes per
 // query (one-wave workgroups) 16.0 us fp16, 19.0 bf16; 8 lanes 15.2; 16 lanes
-// 13.7; this 13.2 and 14.2.
+// 13.7; this 13.2 and 14.2 (13.8 and 14.6 with the V rows of steps without a key
+// cleared).
 constexpr int kMergeParents = 256;
 template <typename T, int D, int WALK, bool BATCH, bool DBG = false>
 __global__ __launch_bounds__(kThreads) void tree_merge_kernel(TreeParams p) {

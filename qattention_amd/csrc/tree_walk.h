@@ -2,8 +2,9 @@
 // kernels (tree_attn.hip) and the fused epilogue of the prefix kernel
 // (prefix_attn.hip).
 //
-// A query (token, q head) is owned by a group of 4 consecutive lanes; lane j
-// holds the 16-byte chunks j, j+4, j+8, ... of every D-element head row (Q, K,
+// A query (token, q head) is owned by a group of 4 consecutive lanes (LPR of
+// them in the group and merge kernels); lane j holds the 16-byte chunks j, j+4,
+// j+8, ... of every D-element head row (Q, K,
 // V rows and the fp32 accumulator), so a chunk of the row is 64 contiguous
 // bytes per group and the dot-product reduction is a 2-step DPP quad sum.
 // Scores are kept in the log2 domain: s = (q . k) * scale * log2(e).
@@ -224,7 +225,8 @@ static __device__ Vec16 kZeroRow[16];  // 128 elements, the widest head
 // self-loop).  A caller may issue the first chunk before it builds the
 // initial state, so those loads overlap its own.
 // DBG (walk export): every step's attended node (or -1) is written to dbg[step].
-// LPR: lanes per row (4, or 8 where the loaded rows serve several queries).
+// LPR: lanes per row (4; 8 where the loaded rows serve several queries, 8 or 16
+// in calls too small to fill the chip).
 template <typename T, int D, int WALK, int LAYOUT, int CH_ = 8 / (D / 32), bool BATCH = false, bool DBG = false,
           int LPR = 4>
 struct Walk4 {

@@ -67,7 +67,7 @@ CASES = [
     ([1025, 1024, 7], 2, 3, 16, 8, 128, torch.float16),
     ([2049, 2050], 5, 6, 32, 8, 32, torch.float16),
     ([2100], 1, 9, 32, 8, 64, torch.float16),
-    # one head per slot: 16 and 8 lanes, at and one node past their limits
+    # one head per slot (16 and 8 lanes) and the gather kernel beyond
     ([512], 2, 9, 32, 32, 128, torch.float16),
     ([513], 2, 9, 32, 32, 128, torch.bfloat16),
     ([256, 0], 4, 4, 16, 8, 128, torch.bfloat16),
@@ -166,7 +166,8 @@ def test_group_strided_and_captured():
     (8, 1023, 2, 9, 32, 8, 128),    # auto: the subtree kernel, deep trees
 ])
 def test_auto_choice_agrees_with_every_kernel(B, N, b, md, Hq, Hkv, D):
-    """The kernel that the estimates choose computes what the others do: two
+    """The kernel that the estimates choose (test_gpu_dispatch.py asserts which)
+    computes what the others do: two
     fp32 softmaxes over the same rounded rows differ by less than one fp16
     rounding of O (2^-10 of |O| <= 6)."""
     ra, _ = _ra()

@@ -460,8 +460,8 @@ def test_paged_subtree_bf16():
 
 
 def test_paged_subtree_table_limit():
-    """A page table of more than 2048 entries: the automatic choice runs the
-    gather kernel (same results), the forced subtree kernel is an error."""
+    """A page table of more than 2048 entries: the automatic choice runs a
+    walk kernel (same results), the forced subtree kernel is an error."""
     ra, lib = _ra()
     say("paged table limit")
     lens, b, md = [121] * 3, 3, 4
@@ -478,8 +478,8 @@ def test_paged_subtree_table_limit():
 
 def test_paged_subtree_needs_equal_strides():
     """The paged subtree kernel addresses K and V with one offset: a V cache
-    with other strides (here every page padded by one slot) runs on the
-    gather kernel under the automatic choice, and is an error when the
+    with other strides (here every page padded by one slot) runs on a
+    walk kernel under the automatic choice, and is an error when the
     subtree kernel is forced."""
     ra, lib = _ra()
     say("paged strides")
