@@ -1,7 +1,8 @@
 """The one-wave-per-query merge and walk: split prefix states of few queries.
 
-It serves split prefix calls of fewer than 8192 (token, q head) pairs.  Cases
-at the sizes where its sharing of states and steps between lane groups can go
+It serves split prefix calls of few (token, q head) pairs (the limits, by head
+size and type, are in test_gpu_dispatch.py; the D = 32 case of 8160 pairs is the
+gather kernel's).  Cases at the sizes where its sharing of states and steps between lane groups can go
 wrong: fewer splits than groups, more than two per group, walks of one step,
 of exactly and more than two rounds of steps, trees on both sides of the 256
 parents kept in registers, empty sequences.  Checked against the fp64 oracle
